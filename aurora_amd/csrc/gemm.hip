@@ -21,6 +21,8 @@
 // tiles that a second kernel reduces in fixed split order — deterministic,
 // no atomics — and adds into the destination.
 #include "common.hpp"
+#include "gemm_split.hpp"
+#include "gemm_tile.hpp"
 
 #include <map>
 #include <mutex>
@@ -29,162 +31,16 @@
 #include <type_traits>
 #include <cstdlib>
 
+using namespace aurgemm;
+
+// Floats of aur_outer_accum_noalloc's scratch array.  The split-fp16 kernel's
+// K ranges are also held to it, so that call and aur_outer_accum, which share
+// one plan, take the same shapes.
+constexpr size_t kNoAllocScratchFloats = size_t(1) << 24;
+
 namespace {
 
 constexpr int kThreads = 256;
-
-struct GemmArgs {
-  const float* A;
-  const float* B;
-  float* C;
-  float* P;  // split-K partials [splits][M][N]
-  int M, N, K;
-  int lda, ldb, ldc;
-  int k_chunk;  // K range per blockIdx.z (multiple of BK)
-  int split;    // 1: write partial tiles to P[z] (epilogue runs in splitk_reduce)
-  int tiles_m, tiles_n;
-  aur::Epilogue epi;
-  // Strided batch (gridDim.y > 1): problem z uses A + z·sA, B + z·sB, C + z·sC.
-  long long sA, sB, sC;
-};
-
-// Points the operands at problem blockIdx.y of a strided batch.
-__device__ __forceinline__ void select_batch(GemmArgs& g) {
-  if (gridDim.y > 1) {
-    const long long z = blockIdx.y;
-    g.A += z * g.sA;
-    g.B += z * g.sB;
-    g.C += z * g.sC;
-  }
-}
-
-// Fused epilogue on one output element v = (A·B)(row, col), stored at C[i]
-// with i = row*ldc + col (R, X, C2 share C's layout).
-// GELU, tanh form (src/linalg.rs:72-87): gelu(x) = 0.5·x·(1 + tanh(u)),
-// u = √(2/π)·(x + 0.044715·x³).  With σ(t) = 1/(1 + e^(−t)) the identities
-// 1 + tanh(u) = 2σ(2u) and sech²(u) = 4σ(2u)(1 − σ(2u)) give both the value
-// and the derivative from one exp2 and one reciprocal, with no cancellation:
-//   gelu(x)  = x·σ(2u)
-//   gelu'(x) = σ(2u) + 2x·σ(2u)(1 − σ(2u))·√(2/π)·(1 + 3·0.044715·x²)
-// (1 − σ(2u) = e^(−2u)·σ(2u) where σ is near 1).  The tanhf form spends
-// most of the FFN GEMM epilogues in VALU work.
-__device__ __forceinline__ float gelu_sigma(float x, float& one_minus) {
-  const float k = 0.7978845608028654f, log2e = 1.4426950408889634f;
-  const float u = k * (x + 0.044715f * x * x * x);
-  const float e = __builtin_amdgcn_exp2f(-2.0f * log2e * u);  // e^(−2u)
-  const float sig = __builtin_amdgcn_rcpf(1.0f + e);
-  one_minus = e < 1.0f ? e * sig : 1.0f - sig;
-  return sig;
-}
-
-__device__ __forceinline__ float gelu_tanh(float x) {
-  float om;
-  return x * gelu_sigma(x, om);
-}
-
-__device__ __forceinline__ float gelu_tanh_grad(float x) {
-  const float k = 0.7978845608028654f;
-  float om;
-  const float sig = gelu_sigma(x, om);
-  return sig + 2.0f * x * sig * om * (k * (1.0f + 3.0f * 0.044715f * x * x));
-}
-
-__device__ __forceinline__ void apply_epilogue(const aur::Epilogue& e, float* __restrict__ C, size_t i,
-                                               float v) {
-  switch (e.mode) {
-    case aur::EPI_ACCUM: C[i] = C[i] + v; break;
-    case aur::EPI_RESID: C[i] = e.R[i] + v; break;
-    case aur::EPI_GELU:
-      C[i] = v;
-      e.C2[i] = gelu_tanh(v);
-      break;
-    case aur::EPI_GELU_BWD: C[i] = v * gelu_tanh_grad(e.X[i]); break;
-    default: C[i] = v; break;
-  }
-}
-
-// Writes a wave's TM×TN grid of 16×16 accumulator tiles (lane holds rows
-// 4·g16 + e, column l16 of each) with the epilogue mode fixed at compile
-// time, so the store loops carry no per-element branch.  MODE −1: split-K
-// partial tile into P[z].  `full`: every row and column is in range.
-template <int MODE, int TM, int TN>
-__device__ __forceinline__ void write_tile(const GemmArgs& g, const floatx4 (&acc)[TM][TN], int r0, int c0,
-                                           int g16, int l16, bool full) {
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int col = c0 + j * 16 + l16;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = r0 + i * 16 + 4 * g16 + e;
-        if (!full && (row >= g.M || col >= g.N)) continue;
-        const float v = acc[i][j][e];
-        if constexpr (MODE < 0) {
-          g.P[((size_t)blockIdx.z * g.M + row) * g.N + col] = v;
-        } else {
-          const size_t idx = (size_t)row * g.ldc + col;
-          if constexpr (MODE == aur::EPI_ACCUM) g.C[idx] = g.C[idx] + v;
-          else if constexpr (MODE == aur::EPI_RESID) g.C[idx] = g.epi.R[idx] + v;
-          else if constexpr (MODE == aur::EPI_GELU) {
-            g.C[idx] = v;
-            g.epi.C2[idx] = gelu_tanh(v);
-          } else if constexpr (MODE == aur::EPI_GELU_BWD) g.C[idx] = v * gelu_tanh_grad(g.epi.X[idx]);
-          else g.C[idx] = v;
-        }
-      }
-    }
-}
-
-template <int TM, int TN>
-__device__ __forceinline__ void write_tiles(const GemmArgs& g, const floatx4 (&acc)[TM][TN], int r0, int c0,
-                                            int g16, int l16, bool full) {
-  if (g.split) {
-    write_tile<-1>(g, acc, r0, c0, g16, l16, full);
-    return;
-  }
-  switch (g.epi.mode) {
-    case aur::EPI_ACCUM: write_tile<aur::EPI_ACCUM>(g, acc, r0, c0, g16, l16, full); break;
-    case aur::EPI_RESID: write_tile<aur::EPI_RESID>(g, acc, r0, c0, g16, l16, full); break;
-    case aur::EPI_GELU: write_tile<aur::EPI_GELU>(g, acc, r0, c0, g16, l16, full); break;
-    case aur::EPI_GELU_BWD: write_tile<aur::EPI_GELU_BWD>(g, acc, r0, c0, g16, l16, full); break;
-    default: write_tile<aur::EPI_STORE>(g, acc, r0, c0, g16, l16, full); break;
-  }
-}
-
-// The epilogue operand (R or X, laid out like C) of a wave's TM×TN tiles,
-// in the accumulator layout: pre[i][j][e] = S[r0 + 16i + 4·g16 + e][c0 + 16j + l16].
-template <int TM, int TN>
-__device__ __forceinline__ void load_epi_operand(const GemmArgs& g, floatx4 (&pre)[TM][TN], int r0, int c0,
-                                                 int g16, int l16, int mode) {
-  const float* src = mode == aur::EPI_RESID ? g.epi.R : g.epi.X;
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        pre[i][j][e] = src[(size_t)(r0 + i * 16 + 4 * g16 + e) * g.ldc + c0 + j * 16 + l16];
-}
-
-// write_tile for whole tiles whose epilogue operand was prefetched.
-template <int MODE, int TM, int TN>
-__device__ __forceinline__ void write_tile_pre(const GemmArgs& g, const floatx4 (&acc)[TM][TN],
-                                               const floatx4 (&pre)[TM][TN], int r0, int c0, int g16,
-                                               int l16) {
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const size_t idx = (size_t)(r0 + i * 16 + 4 * g16 + e) * g.ldc + c0 + j * 16 + l16;
-        if constexpr (MODE == aur::EPI_RESID)
-          g.C[idx] = pre[i][j][e] + acc[i][j][e];
-        else
-          g.C[idx] = acc[i][j][e] * gelu_tanh_grad(pre[i][j][e]);
-      }
-}
 
 template <int BM, int BN, int BK, bool AK, bool BKC>
 struct Smem {
@@ -960,36 +816,81 @@ __global__ void __launch_bounds__(256) stream_partials_kernel(GemmArgs g) {
 
 struct Plan {
   int bm, bn, splits, k_chunk;
+  bool f16 = false;       // the split-fp16 kernel (gemm_split.hip)
+  int fp32_splits = 1;    // K ranges of the plan that the fp32 kernels would have
 };
 
 constexpr int kBK = 32;
 
-// Launch plan: tile shape and split-K count, chosen by a time model.  Blocks
-// are spread over the CUs, so the busiest CU runs L = ceil(blocks / CUs)
-// blocks of f = 2·BM·BN·k_chunk FLOP each, at the CU's peak (256 FLOP/clk)
-// times the tile's relative MFMA efficiency, and slower still when the CU
-// holds a single block (one wave per SIMD leaves LDS and barrier latency
-// exposed).  Split-K adds its reduction pass: the partial planes, the output
-// and any epilogue operand (extra_planes) through HBM, plus one launch.
-// Splits keep ≥ 512 of K per block.  The lowest modelled time wins, ties
-// going to the larger tile and fewer splits.  The constants are fitted on
-// MI355X to every forced configuration (6 tiles × split-K 1…16) of 50
-// shapes — the config-1 and config-3 GEMMs of all three forms at M = 8192 /
-// 16384 and at one GPU's 8-way data-parallel share, M = 1024 / 2048 — timed
-// by `bench.py --only planner`: tile efficiency 1.00 / 0.95 / 0.90 / 0.70 /
-// 0.55 (128×128 / 128×64 / 64×64 / 64×32 / 32×32), single-block factor 0.95
-// / 0.95 / 0.85 / 0.7 / 0.7 (the software-pipelined main loop keeps one
-// wave per SIMD nearly as busy as two), 3 TB/s for the reduction and 2 µs
-// per launch; on the fitting run the pick was within 1.6 % of the measured
-// best on every shape (0.15 % on average).  The two small tiles serve
-// few-tile shapes (M = 1024 with N = 512: 24 → 38 % of peak).
+// What choose_plan may use and what it has to know of a product.
+struct PlanOpts {
+  bool allow_split = true;
+  int batch = 1;
+  int extra_planes = 0;     // epilogue operands the split-K reduction reads
+  bool wide = false;        // the 256×128 fp32 tile may run
+  bool vec = true;          // the fp32 kernels may use 16-byte loads
+  bool f16 = false;         // the split-fp16 kernel may run
+  bool f16_split = true;    // … with several K ranges
+  int k_strided = 0;        // k-strided operands: 0, 1 or 2
+};
+
+// Time of the split-fp16 kernel on `blocks` blocks of nk stages (32 of K)
+// each.  A CU holds `resident` blocks at once; `per_stage` is its time per
+// stage and block with that many, `alone` the time a stage takes at least,
+// however few blocks share the CU, `fixed` a round's prologue, epilogue and
+// fill, `strided` the factor when both operands are k-strided (half of it for
+// one).  Fitted on MI355X to every tile × split-K 1…16 of 100 shapes (the
+// configuration-1 and -3 layers of all three forms, their 8-way shares,
+// d_model 128…512 layers and 40 drawn ones, M 64…16384, K 64…16384, odd sizes
+// among them): 9 % rms error of the time, and the pick is on average 1 %
+// slower than the best forced one.
+struct SplitTile {
+  int bm, bn, resident;
+  double fixed, per_stage, alone, strided;  // µs
+};
+constexpr SplitTile kSplitTiles[] = {{256, 256, 1, 11.1, 2.17, 2.17, 1.11},
+                                     {256, 128, 1, 5.8, 1.31, 1.31, 1.19},
+                                     {128, 128, 2, 4.6, 0.78, 1.02, 1.23},
+                                     {64, 64, 4, 1.53, 0.30, 0.52, 1.22}};
+
+double split_tile_us(const SplitTile& t, long blocks, int cus, int nk, int k_strided) {
+  const long per_cu = (blocks + cus - 1) / cus, full = per_cu / t.resident, rem = per_cu % t.resident;
+  const double form = 1.0 + (t.strided - 1.0) * k_strided / 2;
+  const double stage = full * std::max(t.alone, t.resident * t.per_stage) +
+                       (rem ? std::max(t.alone, rem * t.per_stage) : 0.0);
+  return 3.5 + t.fixed * (full + (rem ? 1 : 0)) + nk * form * stage;
+}
+
+// Launch plan: kernel, tile shape and split-K count, chosen by a time model.
 //
-// allow_wide admits the 256×128 tile (direct-load kernel only: whole tiles,
-// aligned operands, A k-contiguous — with A k-strided it measured 4 % slower
-// than 128×128 — and no prefetched epilogue operand): 1.03 relative
-// efficiency (NT 8192×8192×512: 135.8 vs 130.7 TFLOP/s), 0.75 when alone on a CU.
-Plan choose_plan(const aur_ctx* ctx, int M, int N, int K, bool allow_split, int batch = 1,
-                 int extra_planes = 0, bool allow_wide = false) {
+// fp32 MFMA kernels: blocks are spread over the CUs, so the busiest CU runs
+// L = ceil(blocks / CUs) blocks of f = 2·BM·BN·k_chunk FLOP each, at the CU's
+// peak (256 FLOP/clk) times the tile's relative MFMA efficiency, and slower
+// still when the CU holds a single block (one wave per SIMD leaves LDS and
+// barrier latency exposed).  Split-K adds its reduction pass: the partial
+// planes, the output and any epilogue operand (extra_planes) through HBM, plus
+// one launch.  Splits keep ≥ 512 of K per block.  The lowest modelled time
+// wins, ties going to the larger tile and fewer splits.  The constants are
+// fitted on MI355X to every forced configuration (6 tiles × split-K 1…16) of
+// 50 shapes: tile efficiency 1.00 / 0.95 / 0.90 / 0.70 / 0.55 (128×128 /
+// 128×64 / 64×64 / 64×32 / 32×32), single-block factor 0.95 / 0.95 / 0.85 /
+// 0.7 / 0.7 (the software-pipelined main loop keeps one wave per SIMD nearly
+// as busy as two), 3 TB/s for the reduction and 2 µs per launch.  `wide`
+// admits the 256×128 tile (direct-load kernel only: whole tiles, aligned
+// operands, A k-contiguous — with A k-strided it measured 4 % slower than
+// 128×128 — and no prefetched epilogue operand): 1.03 relative efficiency,
+// 0.75 when alone on a CU.  Against the clock the modelled time stands for
+// 2.1 µs + 1.17 × it on whole tiles, 1.23 × with edges, 2.3 × where the rows
+// allow no 16-byte loads (12 % rms on the same 100 shapes).
+//
+// The split-fp16 kernel (≥ 128 of K per block) takes over where its modelled
+// time is below 0.88 of the fp32 kernels': the margin covers both models'
+// errors, so a call near the line (few tiles or a short K, where launch and
+// latency decide, e.g. 1024×256×1024: 10.1 µs fp32, 12.5 split) stays with
+// the fp32 kernels.  16384×1024×4096: 970 → 390 µs, 8192×2048×512: 129 → 59.
+// Below K = 64 its error no longer has a clear margin under the fp32 MFMA's,
+// so the fp32 kernels keep those.
+Plan choose_plan(const aur_ctx* ctx, int M, int N, int K, const PlanOpts& o) {
   const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
   constexpr double kCuFlops = 256.0 * 2.4e9;  // FLOP/s per CU, fp32 MFMA
   constexpr double kHbm = 3.0e12, kLaunch = 2.0e-6;
@@ -1002,10 +903,10 @@ Plan choose_plan(const aur_ctx* ctx, int M, int N, int K, bool allow_split, int 
   Plan p{128, 128, 1, K};
   double best = 1e30;
   for (const Cand& c : cands) {
-    if (c.bm == 256 && !allow_wide) continue;
-    const long tiles = (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * batch;
+    if (c.bm == 256 && !o.wide) continue;
+    const long tiles = (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * o.batch;
     for (int s = 1; s <= 16; s *= 2) {
-      if (s > 1 && (!allow_split || K / s < 512)) break;
+      if (s > 1 && (!o.allow_split || K / s < 512)) break;
       int chunk = (K + s - 1) / s;
       chunk = (chunk + kBK - 1) / kBK * kBK;
       const int splits = (K + chunk - 1) / chunk;
@@ -1013,27 +914,51 @@ Plan choose_plan(const aur_ctx* ctx, int M, int N, int K, bool allow_split, int 
       const long per_cu = (blocks + cus - 1) / cus;
       const double f = 2.0 * c.bm * c.bn * chunk;
       double t = per_cu * f / (kCuFlops * c.eff * (per_cu == 1 ? c.single : 1.0));
-      if (splits > 1) t += (splits + 1.0 + extra_planes) * M * N * 4.0 * batch / kHbm + kLaunch;
+      if (splits > 1) t += (splits + 1.0 + o.extra_planes) * M * N * 4.0 * o.batch / kHbm + kLaunch;
       if (t < best * (1.0 - 1e-9)) {
         best = t;
         p = {c.bm, c.bn, splits, chunk};
       }
     }
   }
-  // Tuning override: AUR_GEMM_CFG="BMxBN[:splits]".
+  p.fp32_splits = p.splits;
+  if (o.f16 && K >= 64) {
+    const bool whole = o.vec && M % 32 == 0 && N % 32 == 0 && K % 32 == 0;
+    double best_us = 0.88 * (2.1 + 1e6 * best * (whole ? 1.17 : o.vec ? 1.23 : 2.3));
+    for (const SplitTile& c : kSplitTiles) {
+      const long tiles = (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * o.batch;
+      for (int s = 1; s <= 16; s *= 2) {
+        if (s > 1 && (!o.allow_split || !o.f16_split || K / s < 128)) break;
+        int chunk = (K + s - 1) / s;
+        chunk = (chunk + kBK - 1) / kBK * kBK;
+        const int splits = (K + chunk - 1) / chunk;
+        if (splits > 1 && (size_t)splits * M * N > kNoAllocScratchFloats) break;
+        double t = split_tile_us(c, tiles * splits, cus, chunk / kBK, o.k_strided);
+        if (splits > 1) t += 2.2 + (splits + 1.0 + o.extra_planes) * M * N * 4.0 * o.batch / 4.0e6;
+        if (t < best_us * (1.0 - 1e-9)) {
+          best_us = t;
+          p = {c.bm, c.bn, splits, chunk, true, p.fp32_splits};
+        }
+      }
+    }
+  }
+  // Tuning override: AUR_GEMM_CFG="[h]BMxBN[:splits]" (h: the split-fp16 kernel).
   if (const char* env = std::getenv("AUR_GEMM_CFG")) {
     int bm = 0, bn = 0, sp = 1;
-    if (std::sscanf(env, "%dx%d:%d", &bm, &bn, &sp) >= 2 &&
-        ((bm == 128 && bn == 128) || (bm == 128 && bn == 64) || (bm == 64 && bn == 64) ||
-         (bm == 64 && bn == 32) || (bm == 32 && bn == 32) || (bm == 256 && bn == 128 && allow_wide))) {
+    const bool f16 = env[0] == 'h';
+    if (std::sscanf(env + f16, "%dx%d:%d", &bm, &bn, &sp) >= 2 &&
+        (f16 ? o.f16 && ((bm == 256 && (bn == 256 || bn == 128)) || (bm == 128 && bn == 128) || (bm == 64 && bn == 64)) :
+         (bm == 128 && bn == 128) || (bm == 128 && bn == 64) || (bm == 64 && bn == 64) ||
+         (bm == 64 && bn == 32) || (bm == 32 && bn == 32) || (bm == 256 && bn == 128 && o.wide))) {
       p.bm = bm;
       p.bn = bn;
-      if (!allow_split) sp = 1;
+      if (!o.allow_split) sp = 1;
       sp = std::max(1, sp);
       int chunk = (K + sp - 1) / sp;
       chunk = (chunk + kBK - 1) / kBK * kBK;
       p.splits = std::max(1, (K + chunk - 1) / chunk);
       p.k_chunk = chunk;
+      p.f16 = f16;
     }
   }
   return p;
@@ -1100,6 +1025,13 @@ void launch_layout(const GemmArgs& a, const Plan& p, bool vec, hipStream_t st, i
     launch_tile<32, 32, AK, BKC>(a, p.splits, vec, st, batch, cus);
 }
 
+// What the split-fp16 kernel's addressing takes: a thread's rows lie within 32
+// bits of the tile's origin, and its column pairs need an extent of two.  No
+// alignment is asked of the operands.
+bool split_kernel_takes(int M, int N, int lda, int ldb) {
+  return M >= 2 && N >= 2 && lda < (1 << 21) && ldb < (1 << 21);
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 }  // namespace
@@ -1109,7 +1041,6 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 // process ends.  Host code never uses this name as an address (on the host it
 // is only a stand-in for the symbol): it takes each device's address from
 // hipGetSymbolAddress once, at aur_init, and passes that to the kernels.
-constexpr size_t kNoAllocScratchFloats = size_t(1) << 24;
 static __device__ __align__(256) float scratch[kNoAllocScratchFloats];
 
 namespace aur {
@@ -1259,7 +1190,23 @@ int gemm(aur_ctx* ctx, bool a_kcontig, bool b_kcontig, const float* A, int lda, 
   const bool wide = vec && a_kcontig && M % 256 == 0 && N % 128 == 0 && K % 32 == 0 &&
                     epi.mode != EPI_RESID && epi.mode != EPI_GELU_BWD &&
                     std::getenv("AUR_GEMM_STAGED") == nullptr;
-  Plan p = choose_plan(ctx, M, N, K, /*allow_split=*/true, 1, epi.mode == EPI_STORE ? 0 : 1, wide);
+  PlanOpts o;
+  o.extra_planes = epi.mode == EPI_STORE ? 0 : 1;
+  o.wide = wide;
+  o.vec = vec;
+  o.f16 = split_kernel_takes(M, N, lda, ldb);
+  o.k_strided = !a_kcontig + !b_kcontig;
+  Plan p = choose_plan(ctx, M, N, K, o);
+  if (p.f16 && p.splits > 1 && p.fp32_splits == 1 && !(ws && ws->ptr)) {
+    // Being captured, this product could not use the context's workspace (see
+    // partials), and the fp32 kernels would not have needed any: one K range.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    AUR_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cap));
+    if (cap != hipStreamCaptureStatusNone) {
+      o.f16_split = false;
+      p = choose_plan(ctx, M, N, K, o);
+    }
+  }
   GemmArgs a{};
   a.A = A;
   a.B = B;
@@ -1274,12 +1221,16 @@ int gemm(aur_ctx* ctx, bool a_kcontig, bool b_kcontig, const float* A, int lda, 
   a.tiles_n = (N + p.bn - 1) / p.bn;
   a.k_chunk = p.k_chunk;
   a.epi = epi;
-  if (p.splits > 1) {
-    int rc = partials(ctx, ws, (size_t)p.splits * M * N, &a.P);
+  if (std::max(p.splits, p.fp32_splits) > 1) {
+    // Sized (and refused) for the fp32 plan too, so the route taken does not
+    // change which calls a given workspace or a capture admits.
+    int rc = partials(ctx, ws, (size_t)std::max(p.splits, p.fp32_splits) * M * N, &a.P);
     if (rc) return rc;
-    a.split = 1;
+    a.split = p.splits > 1;
   }
-  if (a_kcontig && b_kcontig)
+  if (p.f16)
+    gemm_split_launch(a, p.bm, p.bn, a_kcontig, b_kcontig, p.splits, 1, ctx->stream);
+  else if (a_kcontig && b_kcontig)
     launch_layout<true, true>(a, p, vec, ctx->stream, ctx->cu_count);
   else if (a_kcontig && !b_kcontig)
     launch_layout<true, false>(a, p, vec, ctx->stream, ctx->cu_count);
@@ -1314,7 +1265,14 @@ int gemm_batched(aur_ctx* ctx, bool a_kcontig, bool b_kcontig, const float* A, i
                    (b_kcontig ? (K % 4 == 0) : (N % 4 == 0));
   const bool wide = vec && a_kcontig && M % 256 == 0 && N % 128 == 0 && K % 32 == 0 &&
                     std::getenv("AUR_GEMM_STAGED") == nullptr;
-  const Plan p = choose_plan(ctx, M, N, K, /*allow_split=*/false, batch, 0, wide);
+  PlanOpts o;
+  o.allow_split = false;
+  o.batch = batch;
+  o.wide = wide;
+  o.vec = vec;
+  o.f16 = split_kernel_takes(M, N, lda, ldb);
+  o.k_strided = !a_kcontig + !b_kcontig;
+  const Plan p = choose_plan(ctx, M, N, K, o);
   GemmArgs a{};
   a.A = A; a.B = B; a.C = C; a.M = M; a.N = N; a.K = K;
   a.lda = lda; a.ldb = ldb; a.ldc = ldc;
@@ -1322,7 +1280,9 @@ int gemm_batched(aur_ctx* ctx, bool a_kcontig, bool b_kcontig, const float* A, i
   a.tiles_n = (N + p.bn - 1) / p.bn;
   a.k_chunk = p.k_chunk;
   a.sA = sA; a.sB = sB; a.sC = sC;
-  if (a_kcontig && b_kcontig)
+  if (p.f16)
+    gemm_split_launch(a, p.bm, p.bn, a_kcontig, b_kcontig, 1, batch, ctx->stream);
+  else if (a_kcontig && b_kcontig)
     launch_layout<true, true>(a, p, vec, ctx->stream, ctx->cu_count, batch);
   else if (a_kcontig && !b_kcontig)
     launch_layout<true, false>(a, p, vec, ctx->stream, ctx->cu_count, batch);

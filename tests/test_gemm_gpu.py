@@ -427,3 +427,117 @@ def test_gemm_ex_rejects_short_leading_dimensions(ctx):
         x.free()
     cw, fr = _gates(got, a.reshape(m, k).astype(np.float64), b.reshape(n, k).T.astype(np.float64))
     assert cw < TOL_GEMM and fr < TOL_GEMM, (cw, fr)
+
+
+# ---- the split-fp16 kernel (gemm_split.hip), every tile forced
+
+
+def _split_ex(ctx, monkeypatch, cfg, a, b, ak, bk, splits=1):
+    """op(A)·op(B) of float32 [m, k] and [k, n] arrays through aur_gemm_ex, the
+    operands stored with the given orders and a leading dimension one longer
+    than the row (so that no row is 16-byte aligned)."""
+    from aurora_amd.gpu import GpuBuffer
+
+    def stored(x):
+        s = np.full((x.shape[0], x.shape[1] + 1), 7.0, np.float32)
+        s[:, :-1] = x
+        return s.ravel()[:-1]  # the buffer ends with the last element
+
+    (m, k), n = a.shape, b.shape[1]
+    monkeypatch.setenv("AUR_GEMM_CFG", f"{cfg}:{splits}")
+    ab = GpuBuffer.from_slice(ctx, stored(a if ak else a.T))
+    bb = GpuBuffer.from_slice(ctx, stored(b.T if bk else b))
+    cb = GpuBuffer.zeros(ctx, m * n)
+    ctx.call("aur_gemm_ex", ak, bk, ab.ptr, (k if ak else m) + 1, bb.ptr, (k if bk else n) + 1, cb.ptr, n, m, n, k, 0)
+    out = cb.download().reshape(m, n)
+    for x in (ab, bb, cb):
+        x.free()
+    monkeypatch.delenv("AUR_GEMM_CFG")
+    return out
+
+
+SPLIT_TILES = ["h256x256", "h256x128", "h128x128", "h64x64"]
+
+
+@pytest.mark.parametrize("cfg", SPLIT_TILES)
+@pytest.mark.parametrize("ak,bk", [(1, 1), (1, 0), (0, 1), (0, 0)])
+def test_split_kernel_edges(ctx, monkeypatch, cfg, ak, bk):
+    """One row or column short of, at and past the tiles, K with every kind of
+    partial last stage (32 k), one and several stages.  Bound per element, in
+    units of (|A||B|)_ij: 2·2^-23.5 from the operands' splits and 2^-22 from the
+    dropped product, one rounding of 2^-24 per 32 products and per addition of
+    them: below (9 + K/32)·2^-24 ≤ 1e-6 for the K here."""
+    bm, bn = (int(x) for x in cfg[1:].split("x"))
+    rng = np.random.default_rng(1000 * ak + 10 * bk + bm)
+    for m, n, k in [(bm - 1, bn + 1, 32), (bm, bn, 64), (bm + 1, bn - 1, 33), (65, 3, 127), (2, 65, 96),
+                    (66, 67, 200), (bm + 63, 2 * bn, 31)]:
+        k = max(k, 64) if k < 32 else k
+        a = rng.standard_normal((m, k)).astype(np.float32)
+        b = rng.standard_normal((k, n)).astype(np.float32)
+        got = _split_ex(ctx, monkeypatch, cfg, a, b, ak, bk)
+        cw, fr = _gates(got, a.astype(np.float64), b.astype(np.float64))
+        assert cw < 1e-6 and fr < 4e-7, (cfg, ak, bk, m, n, k, cw, fr)
+
+
+@pytest.mark.parametrize("cfg", SPLIT_TILES)
+@pytest.mark.parametrize("ak,bk", [(1, 1), (0, 0)])
+def test_split_kernel_scales(ctx, monkeypatch, cfg, ak, bk):
+    """Rows and columns whose magnitude grows along K by up to 2^60 (their scale
+    is lowered while the sum runs), starts with zeros, is tiny (2^-130) or huge
+    (2^100): the error stays at 2^-20 of ‖row of A‖·‖column of B‖, element by
+    element (the split's 2^-38 of the largest value is far below it)."""
+    m, n, k = 130, 140, 333
+    rng = np.random.default_rng(3)
+    a = rng.standard_normal((m, k))
+    b = rng.standard_normal((k, n))
+    t = np.arange(k)
+    a[1::7] *= 2.0 ** (60.0 * t / k - 30)
+    a[2::7, :100] = 0
+    a[3::7] *= 2.0 ** -130
+    a[4::7, rng.integers(0, k, a[4::7].shape[0])] = 4096.0
+    a[5::7] = 0
+    b[:, 1::5] *= (2.0 ** (40.0 * t / k - 20))[:, None]
+    b[:70, 2::5] = 0
+    b[:, 3::5] *= 2.0 ** 30
+    a, b = a.astype(np.float32), b.astype(np.float32)
+    a[6::7] *= np.float32(2.0 ** 60)
+    for splits in (1, 2):
+        got = _split_ex(ctx, monkeypatch, cfg, a, b, ak, bk, splits).astype(np.float64)
+        a64, b64 = a.astype(np.float64), b.astype(np.float64)
+        bound = np.linalg.norm(a64, axis=1)[:, None] * np.linalg.norm(b64, axis=0)[None, :]
+        err = np.abs(got - a64 @ b64)
+        # below 2^-126 a float itself has an absolute spacing of 2^-149
+        assert np.all(err <= 2.0 ** -20 * bound + 2.0 ** -148), (cfg, splits, np.max(err / np.maximum(bound, 1e-300)))
+
+
+@pytest.mark.parametrize("cfg", SPLIT_TILES)
+def test_split_kernel_non_finite(ctx, monkeypatch, cfg):
+    """Infinities and NaN come out as the fp32 MFMA kernels give them, and the
+    finite results beside them stay accurate.  In the rows whose partial sums
+    overflow fp32 (where the fp32 kernels give an infinity or NaN even if the
+    whole sum is in range) a result is either not finite there too or right."""
+    m, n, k = 150, 133, 100
+    rng = np.random.default_rng(4)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    b = rng.standard_normal((k, n)).astype(np.float32)
+    a[3, 40], a[20, 99], a[77, 0], a[140, 5] = np.inf, -np.inf, np.nan, np.inf
+    b[5, 9] = 0.0            # inf · 0 in row 140
+    b[70, 100] = np.inf
+    a[90] = 3e38             # overflows in the sum
+    a[5, :] = np.float32(3.0e38)
+    b[:, 11] = 1.0
+    for ak, bk in [(1, 1), (0, 0)]:
+        got = _split_ex(ctx, monkeypatch, cfg, a, b, ak, bk)
+        want = _split_ex(ctx, monkeypatch, "64x64", a, b, ak, bk)
+        plain = [i for i in range(m) if i not in (5, 90)]
+        for kind in (np.isnan, np.isposinf, np.isneginf):
+            assert np.array_equal(kind(got[plain]), kind(want[plain])), (cfg, kind)
+        for i in (5, 90):
+            c64 = a[i].astype(np.float64) @ np.where(np.isfinite(b), b, 0).astype(np.float64)
+            fin = np.isfinite(got[i])
+            assert not np.any(np.isfinite(want[i]) & ~fin)
+            assert np.all(np.abs(got[i][fin] - c64[fin]) <= 1e-6 * 3e38 * np.abs(b[:, fin]).sum(0))
+        rows = [i for i in range(m) if i not in (3, 20, 77, 140, 90, 5)]
+        cols = [j for j in range(n) if j != 100]
+        c64 = a[rows].astype(np.float64) @ b[:, cols].astype(np.float64)
+        assert fro_rel(got[np.ix_(rows, cols)], c64) < 4e-7
