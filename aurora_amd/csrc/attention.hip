@@ -26,62 +26,15 @@
 // reduced over the four 16-lane groups with gfx950's row-swap permutes.
 // The head dimension is covered in chunks of 16 (NC = ceil(DH/16)); when
 // DH is not a multiple of 16 the last chunk's upper half (8 columns) is zero.
+#include "attention.hpp"
 #include "common.hpp"
 
 #include <algorithm>
 #include <cstdlib>
 
+using namespace aurattn;
+
 namespace {
-
-constexpr int TQ = 64;  // rows per tile (4 waves × 16)
-constexpr float LOG2E = 1.4426950408889634f;
-
-struct AttnArgs {
-  const float* q;
-  const float* k;
-  const float* v;
-  const float* o;    // forward output (bwd pass 1)
-  const float* dO;   // gradient of the output
-  float* out;        // forward output
-  float* lse;        // [B, H, T]
-  float* D;          // [B, H, T] rowdot
-  float* ds;         // [B, H, ntri] 64×64 dS tiles of the causal lower triangle (ds_slot)
-  int ntri;          // nqt·(nqt+1)/2 tiles per (sequence, head)
-  float* dq;
-  float* dk;
-  float* dv;
-  int ld_qkv;        // row stride of q, k, v
-  int ld_o;          // row stride of out / o / dO
-  int ld_d;          // row stride of dq, dk, dv
-  int T, H;
-  float scale;       // 1/sqrt(d_head)
-  int overwrite;     // backward: store dq/dk/dv instead of accumulating into them
-};
-
-__device__ __forceinline__ float shfl_xor(float v, int m) { return __shfl_xor(v, m, 64); }
-
-// Max and sum over lanes l, l^16, l^32, l^48 (the four 16-lane rows), every
-// lane getting the result.  v_permlane16_swap exchanges the odd rows of its
-// first operand with the even rows of its second (v_permlane32_swap: the
-// upper half with the lower half), so with both operands = v each lane ends
-// up holding its own value and its partner row's: VALU only, no LDS round
-// trip as with a bpermute.  Sums add (r0 + r1) + (r2 + r3) in every lane.
-__device__ __forceinline__ float rows4_max(float v) {
-  const unsigned u = __float_as_uint(v);
-  auto s = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  v = fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1]));
-  const unsigned u2 = __float_as_uint(v);
-  auto t = __builtin_amdgcn_permlane32_swap(u2, u2, false, false);
-  return fmaxf(__uint_as_float(t[0]), __uint_as_float(t[1]));
-}
-__device__ __forceinline__ float rows4_sum(float v) {
-  const unsigned u = __float_as_uint(v);
-  auto s = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  v = __uint_as_float(s[0]) + __uint_as_float(s[1]);
-  const unsigned u2 = __float_as_uint(v);
-  auto t = __builtin_amdgcn_permlane32_swap(u2, u2, false, false);
-  return __uint_as_float(t[0]) + __uint_as_float(t[1]);
-}
 
 template <int DH>
 struct Geo {
@@ -886,6 +839,19 @@ __global__ void __launch_bounds__(256) unpad_heads_kernel(const float* __restric
 
 unsigned pad_grid(size_t n) { return (unsigned)std::min<size_t>((n + 255) / 256, 8192); }
 
+// The split-fp16 forward (attention_split.hip) halves the time where the CUs
+// are shared by several blocks (B16 H8 T1024: d_head 64 152 → 77 µs, 56 180 →
+// 82, 40 134 → 78, 32 86 → 56, 16 52 → 46).  With about one block per CU both
+// kernels wait on one block's chain of tiles, which its 128-query blocks do not
+// shorten: it starts to win at 1.25 64-query blocks per CU (16×4 heads of T 300:
+// 17.2 → 16.8 µs; 6×4 of T 333: 16.6 → 18.5), later at narrow heads, whose fp32
+// products are short (9×11 heads of 16, T 192: 6.1 → 9.1), and not at one or two
+// tiles (T 128: 10.3 → 10.8 µs at 16×12 heads of 64).
+bool fwd_takes_split(uint32_t b, uint32_t t, uint32_t n_head, uint32_t d_head) {
+  const size_t blocks = (size_t)b * n_head * ((t + TQ - 1) / TQ);
+  return t > 2 * TQ && blocks >= (d_head <= 16 ? 1024 : 320);
+}
+
 template <int DH>
 void launch_fwd(const AttnArgs& a, int b, hipStream_t st) {
   dim3 grid(a.H, b, (a.T + TQ - 1) / TQ);
@@ -1032,6 +998,9 @@ int aur_mha_fwd_ex(aur_ctx* ctx, const float* q, const float* k, const float* v,
   a.ld_qkv = (int)ld_qkv; a.ld_o = (int)ld_out;
   a.T = (int)t; a.H = (int)n_head;
   a.scale = 1.0f / sqrtf((float)scale_dh);
+  if (fwd_takes_split(b, t, n_head, d_head))
+    fwd_split(a, (int)b, (int)d_head, ctx->stream);
+  else
   switch (d_head) {
     case 8: launch_fwd<8>(a, (int)b, ctx->stream); break;
     case 16: launch_fwd<16>(a, (int)b, ctx->stream); break;

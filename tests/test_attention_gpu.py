@@ -451,3 +451,70 @@ def test_kv_step_any_d_head(ctx, t_total, H, dh, max_len):
     got = _kv_single(ctx, q_new, kh, vh, t_total, H, dh, max_len)
     want = oracle.kv_attend(q_new, kh, vh, t_total, H, dh)
     assert fro_rel(got, want) < TOL_ATTN and max_norm_rel(got, want) < TOL_ATTN
+
+
+# ---- the split-fp16 forward (attention_split.hip): taken at T > 128 with enough blocks
+
+
+def _fwd_bthd(ctx, q, k, v, t, h, dh, b):
+    from aurora_amd.gpu import CausalMhaForwardKernel, GpuBuffer
+
+    bufs = [GpuBuffer.from_slice(ctx, x.ravel()) for x in (q, k, v)]
+    o, lse = GpuBuffer.zeros(ctx, q.size), GpuBuffer.zeros(ctx, b * h * t)
+    CausalMhaForwardKernel.new(ctx).dispatch_into(ctx, *bufs, o, lse, t, h, dh, b=b)
+    out = o.download().reshape(b, t, h, dh), lse.download().reshape(b, h, t)
+    for x in (*bufs, o, lse):
+        x.free()
+    return out
+
+
+@pytest.mark.parametrize("t,h,dh,b", [(129, 8, 64, 16), (191, 7, 64, 16), (256, 6, 64, 14), (257, 5, 56, 16),
+                                      (193, 8, 48, 12), (130, 8, 40, 16), (320, 6, 32, 12), (150, 8, 24, 16),
+                                      (131, 16, 16, 24), (129, 16, 8, 24), (140, 8, 20, 16)])
+def test_split_forward_matches_float64(ctx, t, h, dh, b):
+    """Tiles' edges and every head width.  The splits keep 2^-23.5 of each
+    operand, the scores' rounding reaches P through exp (|S| up to about 20 here:
+    20·2^-23) and the sums round once per 32 keys: below 5e-7 in norm, 2e-5 at
+    lse (|lse| up to 200).  v[3] and k[2] make rows of very different sizes, which
+    are computed again with the fp32 MFMA where a tile's scale would not hold
+    them: every output row is held to 2^-16 of its own norm."""
+    rng = np.random.default_rng(t * 100 + dh)
+    q, k, v = (rng.standard_normal((b, t, h, dh)).astype(np.float32) for _ in range(3))
+    q[0] *= 4
+    k[1, :, :, : dh // 2] *= 2.0 ** -20   # tiny beside the rest of the row
+    k[2, ::3] *= 16                       # keys of very different sizes in a tile
+    v[3] *= np.float32(2.0) ** rng.integers(-30, 30, (t, h, 1)).astype(np.float32)
+    v[4, :64] = 0
+    q[5, 1::2] = 0
+    o, lse = _fwd_bthd(ctx, q, k, v, t, h, dh, b)
+    o64, lse64 = causal_attention_f64(*(x.astype(np.float64) for x in (q, k, v)))
+    e = np.linalg.norm(o - o64, axis=-1) / np.maximum(np.linalg.norm(o64, axis=-1), 1e-30)
+    assert e.max() < 2.0 ** -16, (np.unravel_index(e.argmax(), e.shape), e.max())
+    assert np.max(np.abs(lse - lse64)) < 2e-5
+    rest = slice(6, None)
+    e = np.linalg.norm(o[rest] - o64[rest]) / np.linalg.norm(o64[rest])
+    assert e < 5e-7, e
+
+
+def test_split_forward_non_finite(ctx):
+    """Infinities and NaN reach the same outputs as in the fp32 kernel, which a
+    single head runs."""
+    b, t, h, dh = 16, 200, 6, 64
+    rng = np.random.default_rng(5)
+    q, k, v = (rng.standard_normal((b, t, h, dh)).astype(np.float32) for _ in range(3))
+    k[0, 70, 1, 3] = np.inf
+    k[1, 199, 0, 3] = np.nan
+    v[2, 100, 2, 5] = -np.inf
+    v[3, 5, 3, 6] = np.nan
+    q[4, 33, 4, 0] = np.inf
+    q[5, 150] = 1e30
+    k[5, 20] = 1e30
+    o, lse = _fwd_bthd(ctx, q, k, v, t, h, dh, b)
+    for i, j in [(0, 1), (1, 0), (2, 2), (3, 3), (4, 4), (5, 0), (6, 0)]:
+        one = [x[i : i + 1, :, j : j + 1] for x in (q, k, v)]
+        o1, l1 = _fwd_bthd(ctx, *one, t, 1, dh, 1)
+        for got, want in ((o[i, :, j], o1[0, :, 0]), (lse[i, j], l1[0, 0])):
+            assert np.array_equal(np.isnan(got), np.isnan(want)), (i, j)
+            assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+            f = np.isfinite(want)
+            assert np.allclose(got[f], want[f], rtol=2e-5, atol=2e-5)
