@@ -57,5 +57,7 @@ __device__ __forceinline__ float rows4_sum(float v) {
 
 // Forward on the fp16 matrix cores (attention_split.hip), d_head a multiple of 8 up to 64.
 void fwd_split(const AttnArgs& a, int b, int d_head, hipStream_t st);
+// Backward pass 2 (dK, dV and the dS tiles) on them (attention_bwd_split.hip), d_head 24 to 64.
+void bwd_dkv_split(const AttnArgs& a, int b, int d_head, hipStream_t st);
 
 }  // namespace aurattn

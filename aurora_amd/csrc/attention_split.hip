@@ -30,6 +30,7 @@
 // kernel; 16 queries per wave in 8-wave blocks (twice the LDS reads): 93; two
 // LDS stages with one barrier per tile: 78.
 #include "attention.hpp"
+#include "attention_split.hpp"
 #include "common.hpp"
 #include "split16.hpp"
 
@@ -42,31 +43,6 @@ namespace {
 
 constexpr int QB = 128;             // queries per block
 constexpr float kPScale = 16384.f;  // P ≤ 1 is split at this scale
-
-template <int DH>
-struct SplitGeo {
-  static constexpr int KS = (DH + 31) / 32;  // 32-wide steps over the head dimension
-  static constexpr int DT = (DH + 15) / 16;  // 16-row tiles of Vᵀ / Oᵀ
-  static constexpr int KROW = KS * 64;       // bytes of a K row in LDS
-  static constexpr int KPLANE = 64 * KROW, VPLANE = DT * 16 * 128;
-};
-
-// Granule q of row r in rows of 128 bytes: as split_granule, every phase of 16
-// lanes covers the 64 banks once.
-__device__ __forceinline__ int granule128(int r, int q) { return r * 128 + ((q ^ (r >> 1)) & 7) * 16; }
-template <int ROW>
-__device__ __forceinline__ int k_granule(int r, int q) {
-  return ROW == 64 ? split_granule(r, q) : granule128(r, q);
-}
-
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int m = 8; m >= 1; m >>= 1) v = fmaxf(v, shfl_xor(v, m));
-  return rows4_max(v);
-}
-
-// p with max·2^p in [2^13, 2^14).
-__device__ __forceinline__ int tile_exp(float m) { return min(140 - (int)(__float_as_uint(m) >> 23), 127); }
 
 // The 16 queries from q16 of one head again, with the fp32 MFMA and operands
 // straight from memory (see the head of the file).

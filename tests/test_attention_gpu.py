@@ -518,3 +518,69 @@ def test_split_forward_non_finite(ctx):
             assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
             f = np.isfinite(want)
             assert np.allclose(got[f], want[f], rtol=2e-5, atol=2e-5)
+
+
+# ---- the split-fp16 dK/dV pass (attention_bwd_split.hip): taken at T > 128 with enough blocks
+
+
+@pytest.mark.parametrize("t,h,dh,b", [(129, 16, 64, 16), (191, 14, 64, 16), (256, 10, 64, 16), (257, 8, 56, 16),
+                                      (193, 12, 48, 14), (320, 8, 40, 16), (385, 10, 32, 16), (257, 16, 24, 16),
+                                      (300, 8, 36, 16)])
+def test_split_backward_matches_float64(ctx, t, h, dh, b):
+    """Tiles' edges and every head width.  The splits keep 2^-23 of each operand
+    and an error of a score (|S| up to 8 here: a few 2^-21) is a relative one of P
+    and dS: 2e-6 in norm, four times that where |S| is.  Rows of dO of very
+    different sizes go through the fp32 products: every row of dV, a sum with
+    positive weights, is held to 2^-14 of its own norm."""
+    rng = np.random.default_rng(t * 100 + dh)
+    q, k, v, do = (rng.standard_normal((b, t, h, dh)).astype(np.float32) for _ in range(4))
+    q[0] *= 4
+    do[1] *= np.float32(2.0) ** rng.integers(-30, 30, (t, h, 1)).astype(np.float32)
+    do[2, ::2] = 0
+    k[3, :70] = 0
+    q[4] *= 2.0 ** -20
+    do[5] *= 2.0 ** -60
+    q[6, ::5] = 0
+    v[7, :, :, : dh // 2] *= 2.0 ** -18
+    o, lse = _fwd_bthd(ctx, q, k, v, t, h, dh, b)
+    grads = _bwd(ctx, *(x.ravel() for x in (q, k, v, o, lse, do)), b, t, h, dh)
+    g64 = causal_attention_grad_f64(*(x.astype(np.float64) for x in (q, k, v, do)))
+    for name, got, want in zip(("dq", "dk", "dv"), grads, g64):
+        got = got.reshape(b, t, h, dh)
+        for i in range(b):
+            e = np.linalg.norm(got[i] - want[i]) / np.linalg.norm(want[i])
+            assert e < (8e-6 if i == 0 else 2e-6), (name, i, e)
+        if name == "dv":
+            e = np.linalg.norm(got - want, axis=-1) / np.maximum(np.linalg.norm(want, axis=-1), 1e-30)
+            assert e.max() < 2.0 ** -14, (np.unravel_index(e.argmax(), e.shape), e.max())
+
+
+def test_split_backward_non_finite(ctx):
+    """Infinities and NaN reach the same gradients as in the fp32 kernel, which a
+    single head runs; gradients are added to what is there."""
+    b, t, h, dh = 16, 200, 10, 64
+    rng = np.random.default_rng(6)
+    q, k, v, do = (rng.standard_normal((b, t, h, dh)).astype(np.float32) for _ in range(4))
+    k[0, 70, 1, 3] = np.inf
+    k[1, 199, 0, 3] = np.nan
+    v[2, 100, 2, 5] = -np.inf
+    do[3, 5, 3, 6] = np.nan
+    do[4, 130, 4, 0] = np.inf
+    q[5, 150, 0] = 1e30
+    q[6, 180, 1, 2] = np.nan
+    do[7, 199, 2] = 1e38
+    o, lse = _fwd_bthd(ctx, q, k, v, t, h, dh, b)
+    init = rng.standard_normal((3, b, t, h, dh)).astype(np.float32)
+    grads = _bwd(ctx, *(x.ravel() for x in (q, k, v, o, lse, do)), b, t, h, dh, init=[x.ravel() for x in init])
+    for i, j in [(0, 1), (1, 0), (2, 2), (3, 3), (4, 4), (5, 0), (6, 1), (7, 2), (8, 0)]:
+        one = [np.ascontiguousarray(x[i : i + 1, :, j : j + 1]).ravel() for x in (q, k, v, o)]
+        g1 = _bwd(ctx, *one, lse[i, j].ravel(), np.ascontiguousarray(do[i, :, j]).ravel(), 1, t, 1, dh,
+                  init=[np.ascontiguousarray(x[i, :, j]).ravel() for x in init])
+        for name, got, want in zip(("dq", "dk", "dv"), grads, g1):
+            got, want = got.reshape(b, t, h, dh)[i, :, j], want.reshape(t, dh)
+            assert np.array_equal(np.isnan(got), np.isnan(want)), (name, i, j)
+            assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+            f = np.isfinite(want)
+            if f.any():
+                scale = np.abs(want[f]).max()
+                assert np.all(np.abs(got[f] - want[f]) <= 1e-5 * scale), (name, i, j)
