@@ -23,21 +23,35 @@
 //
 // fp16 spans only 2^-24 … 2^16, so every row of A and column of B carries its
 // own power-of-two scale 2^p.  It starts from the row's first 32 values (their
-// largest magnitude goes to 2^7 … 2^8, 128 times below the limit) and shrinks
-// when a later value would pass 2^15; the accumulators of that row are then
-// rescaled (exactly) before the next product is added.  Values far below the
-// row's largest lose relative precision only (their absolute error stays under
-// 2^-38 of it).  A result that is not finite — an infinity or NaN among the
-// operands, or a product that overflows — is recomputed for the wave's whole
-// sub-tile with the fp32 MFMA, so infinities and NaN come out as they do there.
+// largest magnitude goes to 2^13 … 2^14, at least 4 times below the limit) and
+// shrinks when a later value would pass the limit; the accumulators of that row
+// are then rescaled before the next product is added.
+//
+// A value below 2^-2 at that scale, 2^15 … 2^18 below the row's largest, has an
+// absolute error of up to 2^-25 there instead of a relative one, which shows
+// where the row's large values meet zeros or small values of the column.  So the
+// values too small for their scale are counted per row and column (n and m): what
+// they can do to a result is at most E = (n + m)·2^-25·2^16.  It stands if E is
+// below 2^-21 of the sum of the products' magnitudes, for which there are two
+// lower bounds: the result's own magnitude, and, where the first 32 values of row
+// and column hold D and D' of 2^9 or more, (D + D' − 32)·2^18.  (That clears
+// N(0, 1) operands, halves of zeros and GELU outputs without a look at the
+// results.)  The others are computed again in fp32: a few of a wave as dot
+// products, from more on the block's tile with the fp32 MFMA.  So is a tile with a
+// result that is not finite — an infinity or NaN among the operands, or a product
+// that overflows —, so that infinities and NaN come out as they do there.
 //
 // What bounds it: per 32 of K a wave of the 256×256 tile (128×64 outputs)
-// issues 96 MFMAs (1536 matrix-core cycles), 128 additions, ≈ 130 operations
-// of splitting and checking, 24 fragment reads and 8 LDS writes; the matrix
-// cores are busy 55 % of the time and power holds the clock at 1.7-1.9 GHz.
-// Measured (fp32 MFMA kernels → here): A·Bᵀ 16384×1024×4096 970 → 386 µs (355
-// TFLOP/s), 8192×2048×512 129 → 59 µs, dW 4096×1024 over 16384 rows 1016 →
-// 437 µs.  The 256×256 tile needs the fewest LDS and L2 bytes per product; the
+// issues 96 MFMAs (1536 matrix-core cycles), 128 additions, ≈ 150 operations
+// of splitting and checking, 24 fragment reads and 8 LDS writes, and the waves of a
+// SIMD hardly overlap the two; power holds the clock at 1.7-1.9 GHz.
+// Measured (fp32 MFMA kernels → here): A·Bᵀ 16384×1024×4096 970 → 390 µs (352
+// TFLOP/s), 8192×2048×512 129 → 60 µs, dW 4096×1024 over 16384 rows 1016 →
+// 437 µs, 777×1023×513 24.3 → 15.5 µs.  Counting the small values is 2 µs of each
+// but the last's 11 % (one wave per SIMD there).  Tiles that are computed again add
+// the fp32 MFMA's time: 4096×1024×4096 140 µs, all of it again (one outlier of 2^8
+// or more a row, met by zeros) 370 to 440, where the fp32 kernels take 255.
+// The 256×256 tile needs the fewest LDS and L2 bytes per product; the
 // smaller tiles serve shapes with few output tiles (choose_plan in gemm.hip).
 #include "common.hpp"
 #include "gemm_tile.hpp"
@@ -55,13 +69,35 @@ namespace {
 typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
 
-// Scale exponents: p for a row whose first values' largest magnitude is m (0
-// when there is none yet), the lowered p for a row that met a larger m, and
-// the factor 2^p.
-constexpr float kSplitLimit = 32768.f;  // largest scaled magnitude let through
-__device__ __forceinline__ int first_exp(float m) { return min(134 - (int)(__float_as_uint(m) >> 23), 127); }
-__device__ __forceinline__ int lowered_exp(float m) { return 140 - (int)(__float_as_uint(m) >> 23); }
+// Scale exponent p of a row whose largest magnitude is m (0 when there is none
+// yet), and that of the factor 2^p.
+constexpr float kSplitLimit = 65504.f;  // largest scaled magnitude let through
+constexpr float kSplitFine = 0.25f;     // smallest that keeps its 23 bits
+constexpr float kFineBound = 4096.f;    // |result| ≥ this · (n + m), at the scales: E ≤ 2^-21 of it
+constexpr int kDenseBound = 64;         // n + m ≤ this · (D + D' − 32): E ≤ 2^-21 of that bound
+constexpr int kZeroExp = 127;           // of a row of zeros so far, and of no other (but for values below 2^-111)
+__device__ __forceinline__ int row_exp(float m) {
+  return m == 0.f ? kZeroExp : min(140 - (int)(__float_as_uint(m) >> 23), 126);
+}
 __device__ __forceinline__ int scale_exp(float s) { return (int)((__float_as_uint(s) >> 23) & 255) - 127; }
+
+// Byte offset of granule q (4 k) of row r in an fp32 tile [ROWS][32].
+__device__ __forceinline__ int fp32_granule(int r, int q) { return r * 128 + ((q ^ r) & 7) * 16; }
+
+// Is any |h| of the octet outside [kSplitFine, kSplitLimit], zero, infinite or NaN?
+// (2h − 2·0x3400 in 16 bits, without the sign, is below 0x9000 for the others.)
+typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ ushort2v high_range(const half2v (&h)[4]) {
+  ushort2v m = {0, 0};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    ushort2v t;
+    asm("v_pk_mad_u16 %0, %1, 2, %2 op_sel_hi:[1,0,1]" : "=v"(t) : "v"(h[e]), "s"(0x98009800u));
+    m = __builtin_elementwise_max(m, t);
+  }
+  return m;
+}
+__device__ __forceinline__ bool out_of_range(ushort2v t) { return max(t[0], t[1]) >= 0x9000; }
 
 // One operand's share of a thread: NO "octets", each 8 consecutive k of one
 // row (of A, or column of B) in a stage of 32 k.
@@ -157,9 +193,39 @@ struct SplitOperand {
     for (int e = 2; e < 8; e += 2) m = fmaxf(fmaxf(m, fabsf(x[o][e])), fabsf(x[o][e + 1]));
     return m;
   }
+  // Values of octet o that are too small for the row's scale; zeros are exact.
+  __device__ __forceinline__ int octet_fine(int o) const {
+    int n = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) n += (x[o][e] != 0.f) & (fabsf(x[o][e] * s[o]) < kSplitFine);
+    return n;
+  }
+  __device__ __forceinline__ int octet_from(int o, float least) const {
+    int n = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) n += fabsf(x[o][e]) >= least;
+    return n;
+  }
+  // Over a row's four octets (quad permutes, or row and half swaps).
+  template <class Op>
+  __device__ __forceinline__ static int over_row(int v, Op op) {
+    if constexpr (KC) {
+      v = op(v, __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true));
+      return op(v, __builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, true));
+    } else {
+      const auto s = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+      v = op(s[0], s[1]);
+      const auto t = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+      return op(t[0], t[1]);
+    }
+  }
+  __device__ __forceinline__ static int row_sum(int n) {
+    return over_row(n, [](int a, int b) { return a + b; });
+  }
   __device__ __forceinline__ static float row_max(float m) {
-    m = fmaxf(m, __shfl_xor(m, KC ? 1 : 16, 64));
-    return fmaxf(m, __shfl_xor(m, KC ? 2 : 32, 64));
+    return __int_as_float(over_row(__float_as_int(m), [](int a, int b) {
+      return __float_as_int(fmaxf(__int_as_float(a), __int_as_float(b)));
+    }));
   }
   // Odd rows are scaled by −2^p (see the head of the file).
   __device__ __forceinline__ void set_exp(int o, int p) {
@@ -176,50 +242,54 @@ struct SplitOperand {
       }
     }
   }
+  // The high parts of octet o.
+  __device__ __forceinline__ void high(int o, half2v (&h)[4]) const {
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) h[e / 2] = split_high(x[o][e], x[o][e + 1], s[o], s[o]);
+  }
   // h and l of octet o as two 16-byte granules of the LDS planes [ROWS][32].
-  __device__ __forceinline__ void store(int o, char* planes) const {
+  __device__ __forceinline__ void store(int o, const half2v (&hh)[4], char* planes) const {
     half8 h, l;
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
-      half2v hh, ll;
-      split2(x[o][e], x[o][e + 1], s[o], s[o], hh, ll);
-      h[e] = hh[0], h[e + 1] = hh[1];
+      const half2v ll = split_low(x[o][e], x[o][e + 1], s[o], s[o], hh[e / 2]);
+      h[e] = hh[e / 2][0], h[e + 1] = hh[e / 2][1];
       l[e] = ll[0], l[e + 1] = ll[1];
     }
     char* p = planes + lds + step(o) * 64;
     *reinterpret_cast<half8*>(p) = h;
     *reinterpret_cast<half8*>(p + ROWS * 64) = l;
   }
+  // The octets' values as they are, [ROWS][32] floats.
+  __device__ __forceinline__ void store_fp32(char* tile) const {
+#pragma unroll
+    for (int o = 0; o < NO; ++o) {
+      const int r = row0 + step(o), q = koct >> 2;
+      *reinterpret_cast<floatx4*>(tile + fp32_granule(r, q)) = floatx4{x[o][0], x[o][1], x[o][2], x[o][3]};
+      *reinterpret_cast<floatx4*>(tile + fp32_granule(r, q + 1)) = floatx4{x[o][4], x[o][5], x[o][6], x[o][7]};
+    }
+  }
 };
 
-// The wave's sub-tile again with the fp32 MFMA, straight from memory: only for
-// results that are not finite.
-template <int TM, int TN, bool AK, bool BKC>
-__device__ __forceinline__ void fp32_tile(const GemmArgs& g, floatx4 (&acc)[TM][TN], int r0, int c0, int kbeg,
-                                          int kend, int g16, int l16) {
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+// Result (r, c) again in fp32, by the whole wave.
+template <bool AK, bool BKC>
+__device__ __forceinline__ float fp32_dot(const GemmArgs& g, int r, int c, int kbeg, int kend, int lane) {
+  const size_t sa = AK ? 1 : g.lda, sb = BKC ? 1 : g.ldb;
+  const float* pa = g.A + (size_t)r * (AK ? g.lda : 1);
+  const float* pb = g.B + (size_t)c * (BKC ? g.ldb : 1);
+  constexpr int U = 8;
+  float sum[U] = {};
 #pragma unroll 1
-  for (int k0 = kbeg; k0 < kend; k0 += 4) {
-    const int k = k0 + g16;
-    float a[TM], b[TN];
+  for (int k0 = kbeg + lane; k0 < kend; k0 += 64 * U)
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const size_t r = min(r0 + 16 * i + l16, g.M - 1);
-      a[i] = k < kend ? (AK ? g.A[r * g.lda + k] : g.A[(size_t)k * g.lda + r]) : 0.f;
+    for (int i = 0; i < U; ++i) {
+      const int k = k0 + 64 * i;
+      if (k < kend) sum[i] = __builtin_fmaf(pa[k * sa], pb[k * sb], sum[i]);
     }
+  float v = ((sum[0] + sum[1]) + (sum[2] + sum[3])) + ((sum[4] + sum[5]) + (sum[6] + sum[7]));
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const size_t c = min(c0 + 16 * j + l16, g.N - 1);
-      b[j] = k < kend ? (BKC ? g.B[c * g.ldb + k] : g.B[(size_t)k * g.ldb + c]) : 0.f;
-    }
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = mfma16x16x4(a[i], b[j], acc[i][j]);
-  }
+  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+  return v;
 }
 
 // acc += u, at this place: left alone the compiler moves the additions to the
@@ -230,7 +300,7 @@ __device__ __forceinline__ void add_here(floatx4& acc, floatx4 u) {
 }
 
 template <int BM, int BN, int WGM, int WGN, bool AK, bool BKC, bool LATE>
-__global__ void __launch_bounds__(64 * WGM * WGN, 2) gemm_f16x3(GemmArgs g) {
+__global__ void __launch_bounds__(64 * WGM * WGN, BM == 64 ? 4 : 2) gemm_f16x3(GemmArgs g) {
   select_batch(g);
   constexpr int NT = 64 * WGM * WGN;
   constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 16, TN = WN / 16;
@@ -240,6 +310,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) gemm_f16x3(GemmArgs g) {
   // change of the exponent); flag[parity] = the stage that has any.
   __shared__ int2 note[2][BM + BN];
   __shared__ int flag[2];
+  // Of each row of A and column of B: the values too small for their scale; those
+  // of the first 32 that are large (0 once the scale was lowered) + 256·first scale
+  __shared__ int fine[BM + BN], dense[BM + BN];
+  __shared__ int rough;  // a result may have to be looked at
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WGN, wn = wave % WGN;
   const int g16 = lane >> 4, l16 = lane & 15;
@@ -279,18 +353,26 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) gemm_f16x3(GemmArgs g) {
   }
   for (int i = tid; i < 2 * (BM + BN); i += NT) (&note[0][0])[i] = int2{-1, 0};
   if (tid < 2) flag[tid] = -1;
+  if (tid == 0) rough = 0;
+  auto first = [&](auto& op, int o, int note0, char* planes) {
+    op.align(o);
+    const int p = row_exp(op.row_max(op.octet_max(o))), row = note0 + op.row0 + op.step(o);
+    op.set_exp(o, p);
+    half2v h[4];
+    op.high(o, h);
+    op.store(o, h, planes);
+    int n = op.octet_from(o, exp_scale(9 - p));
+    if (__any(out_of_range(high_range(h)))) n |= op.octet_fine(o) << 8;
+    n = op.row_sum(n);
+    if (op.koct == 0) {
+      fine[row] = n >> 8;
+      dense[row] = 256 * p + (n & 255);
+    }
+  };
 #pragma unroll
-  for (int o = 0; o < NOA; ++o) {
-    la.align(o);
-    la.set_exp(o, first_exp(la.row_max(la.octet_max(o))));
-    la.store(o, smem);
-  }
+  for (int o = 0; o < NOA; ++o) first(la, o, 0, smem);
 #pragma unroll
-  for (int o = 0; o < NOB; ++o) {
-    lb.align(o);
-    lb.set_exp(o, first_exp(lb.row_max(lb.octet_max(o))));
-    lb.store(o, smem + BM * 128);
-  }
+  for (int o = 0; o < NOB; ++o) first(lb, o, BM, smem + BM * 128);
   la.advance();
   lb.advance();
   if (nk > 1) {
@@ -306,17 +388,62 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) gemm_f16x3(GemmArgs g) {
   }
   __syncthreads();
 
-  // Octet o of stage kt + 1: its row is rescaled if it passes the limit (rare).
-  auto check = [&](auto& op, int o, int kt, int note0) {
-    op.align(o);
-    const float m = op.octet_max(o);
-    if (__any(m * fabsf(op.s[o]) > kSplitLimit)) {
-      const float rm = op.row_max(m);
-      if (rm * fabsf(op.s[o]) > kSplitLimit) {
-        const int p = lowered_exp(rm);
-        note[(kt + 1) & 1][note0 + op.row0 + op.step(o)] = int2{kt + 1, p - scale_exp(op.s[o])};
-        flag[(kt + 1) & 1] = kt + 1;
-        op.set_exp(o, p);
+  // Octets of stage kt + 1 with values out of range.  A row that passes the limit is
+  // rescaled; values too small for its scale are counted.  What the sums hold may
+  // underflow by a scale 2^60 below the first: that counts as one value.
+  auto rescale = [&](auto& op, int o, int kt, int note0) {
+    const float rm = op.row_max(op.octet_max(o));
+    if (rm * fabsf(op.s[o]) > kSplitLimit) {
+      const int row = note0 + op.row0 + op.step(o), p = row_exp(rm), old = scale_exp(op.s[o]);
+      note[(kt + 1) & 1][row] = int2{kt + 1, p - old};
+      flag[(kt + 1) & 1] = kt + 1;
+      if (op.koct == 0) {
+        const int p0 = old == kZeroExp ? p : dense[row] >> 8;
+        dense[row] = 256 * p0;
+        if (p < p0 - 60) atomicAdd(&fine[row], 1);
+      }
+      op.set_exp(o, p);
+    }
+  };
+  auto count = [&](auto& op, int o, int note0) {
+    const int n = op.octet_fine(o);
+    if (n) atomicAdd(&fine[note0 + op.row0 + op.step(o)], n);
+  };
+  half2v hh[NO][4];  // high parts of the octets to be split next
+  auto high = [&](int o) {
+    if (o < NOA)
+      la.high(o, hh[o]);
+    else
+      lb.high(o - NOA, hh[o]);
+  };
+  ushort2v range;  // of them
+  auto high_octets = [&](int o0, int o1) {
+#pragma unroll
+    for (int o = o0; o < o1; ++o) {
+      if (o < NOA)
+        la.align(o);
+      else
+        lb.align(o - NOA);
+      high(o);
+      range = o == o0 ? high_range(hh[o]) : __builtin_elementwise_max(range, high_range(hh[o]));
+    }
+  };
+  auto check_octets = [&](int o0, int o1, int kt) {
+    if (__any(out_of_range(range))) {
+#pragma unroll
+      for (int o = o0; o < o1; ++o) {
+        const float m = o < NOA ? la.octet_max(o) * fabsf(la.s[o]) : lb.octet_max(o - NOA) * fabsf(lb.s[o - NOA]);
+        if (__any(m > kSplitLimit)) {
+          if (o < NOA)
+            rescale(la, o, kt, 0);
+          else
+            rescale(lb, o - NOA, kt, BM);
+          high(o);
+        }
+        if (o < NOA)
+          count(la, o, 0);
+        else
+          count(lb, o - NOA, BM);
       }
     }
   };
@@ -344,17 +471,20 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) gemm_f16x3(GemmArgs g) {
   // needs of the stage and written its share of the next one, so the last
   // step's MFMAs cover the first fragment reads of the next stage (a column's
   // fragments are replaced as soon as their last MFMA is issued).
+  // An octet's high parts and their range are found under the products of the step
+  // before it by the LATE tile (dx 16384×1024×4096: 390 → 378 µs), at the start of
+  // its own by the others (their registers are loaded too shortly before: 15.6 →
+  // 16.7 µs at 777×1023×513).
+  constexpr int S = TM > 1 ? TM - 1 : 1;  // steps that convert
+  // octets [first_octet(i), first_octet(i + 1)) are split in step i
+  constexpr auto first_octet = [](int i) {
+    if (!LATE) return i * NO / S;
+    return i <= 2 ? 0 : i <= 6 ? NOA : NO;
+  };
   // MODE 0: stage kt + 2 is loaded whole; 1: it is the partial last one; 2:
   // there is none; 3: the last stage, nothing to convert.
   auto step = [&](int kt, auto mode) {
     constexpr int MODE = decltype(mode)::value;
-    constexpr int S = TM > 1 ? TM - 1 : 1;  // steps that convert
-    // octets [first_octet(i), first_octet(i + 1)) are split in step i
-    constexpr auto first_octet = [](int i, int m) {
-      if (m == 3) return 0;
-      if (!LATE) return i * NO / S;
-      return i <= 2 ? 0 : i <= 6 ? NOA : NO;
-    };
     const char* sa = smem + (kt & 1) * STAGE;
     char* na = smem + ((kt + 1) & 1) * STAGE;
     char* nb = na + BM * 128;
@@ -397,21 +527,16 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) gemm_f16x3(GemmArgs g) {
     for (int i = 0; i < TM; ++i) {
       const half8 ch = ah, cl = al;
       if (i + 1 < TM) {
-        const int o0 = first_octet(i, MODE), o1 = first_octet(i + 1, MODE);
-#pragma unroll
-        for (int o = o0; o < o1; ++o) {
-          if (o < NOA)
-            check(la, o, kt, 0);
-          else
-            check(lb, o - NOA, kt, BM);
-        }
+        const int o0 = MODE == 3 ? 0 : first_octet(i), o1 = MODE == 3 ? 0 : first_octet(i + 1);
+        if (!LATE) high_octets(o0, o1);
+        if (o1 > o0) check_octets(o0, o1, kt);
         read_a(sa, i + 1);
 #pragma unroll
         for (int j0 = 0; j0 < TN; j0 += JB) pair(i, j0, ch, cl);
 #pragma unroll
         for (int o = o0; o < o1; ++o) {
           if (o < NOA) {
-            la.store(o, na);
+            la.store(o, hh[o], na);
             if ((o + 1) % la.CV == 0 && MODE < 2 && !LATE) la.template load<MODE == 1>(o / la.CV, ktail);
             if (LATE && o + 1 == NOA) {  // B of stage kt + 1 takes A's registers
               if (MODE == 2 && ktail)
@@ -421,11 +546,12 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) gemm_f16x3(GemmArgs g) {
               lb.advance();
             }
           } else {
-            lb.store(o - NOA, nb);
+            lb.store(o - NOA, hh[o], nb);
             if ((o - NOA + 1) % lb.CV == 0 && MODE < 2 && !LATE) lb.template load<MODE == 1>((o - NOA) / lb.CV, ktail);
             if (LATE && o + 1 == NO && MODE < 2) la.template load_all<MODE == 1>(ktail);  // A of stage kt + 2
           }
         }
+        if (LATE && MODE < 3 && i + 2 < TM) high_octets(first_octet(i + 1), first_octet(i + 2));
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
 #pragma unroll
         for (int r = 0; r < 3 * TN; ++r) {
@@ -468,20 +594,57 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) gemm_f16x3(GemmArgs g) {
   // The rows' and columns' final exponents, through the notes' memory.
   __syncthreads();
   int* ex = reinterpret_cast<int*>(&note[0][0]);
+  // > 0 for a row and a column together: their results are looked at
+  auto doubt = [&](int row) { return fine[row] - kDenseBound * ((dense[row] & 255) - 16); };
+  auto last = [&](auto& op, int o, int note0) {
+    const int row = note0 + op.row0 + op.step(o);
+    if (op.koct == 0) {
+      ex[row] = scale_exp(op.s[o]);
+      if (doubt(row) > 0 && ex[row] != kZeroExp) rough = 1;
+    }
+  };
 #pragma unroll
-  for (int o = 0; o < NOA; ++o)
-    if (la.koct == 0) ex[la.row0 + la.step(o)] = scale_exp(la.s[o]);
+  for (int o = 0; o < NOA; ++o) last(la, o, 0);
 #pragma unroll
-  for (int o = 0; o < NOB; ++o)
-    if (lb.koct == 0) ex[BM + lb.row0 + lb.step(o)] = scale_exp(lb.s[o]);
+  for (int o = 0; o < NOB; ++o) last(lb, o, BM);
   __syncthreads();
   int pc[TN];
-  unsigned worst = 0;
+  // Results to compute again: bit 4j + e of fl[i].
+  unsigned fl[TM], worst = 0;
+  int nfl = 0;
+  if (rough) {
+    // A row or column of zeros, or past the operand, is never in doubt.
+    constexpr int kNever = -(1 << 30);
+    int dc[TN], nc[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int col = BM + wn * WN + 16 * j + l16;
+      nc[j] = fine[col];
+      dc[j] = ex[col] == kZeroExp || n0 + col - BM >= g.N ? kNever : doubt(col);
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      fl[i] = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = wm * WM + 16 * i + 4 * g16 + e, nr = fine[row];
+        const int dr = ex[row] == kZeroExp || m0 + row >= g.M ? kNever : doubt(row);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const float bound = dr + dc[j] > 0 ? kFineBound * (float)(nr + nc[j]) : 0.f;
+          fl[i] |= (fabsf(acc[i][j][e]) < bound ? 1u : 0u) << (4 * j + e);
+        }
+      }
+      nfl += __popc(fl[i]);
+    }
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) nfl += __shfl_xor(nfl, m, 64);
+  }
   const unsigned odd = (unsigned)l16 << 31;
 #pragma unroll
   for (int j = 0; j < TN; ++j) pc[j] = ex[BM + wn * WN + 16 * j + l16];
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int i = 0; i < TM; ++i) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int pr = ex[wm * WM + 16 * i + 4 * g16 + e];
@@ -493,9 +656,91 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) gemm_f16x3(GemmArgs g) {
         worst = max(worst, __float_as_uint(v) & 0x7fffffffu);
       }
     }
+  }
   const int r0 = m0 + wm * WM, c0 = n0 + wn * WN;
-  if (__any(worst >= 0x7f800000u)) fp32_tile<TM, TN, AK, BKC>(g, acc, r0, c0, kbeg, kend, g16, l16);
-  write_tiles(g, acc, r0, c0, g16, l16, m0 + BM <= g.M && n0 + BN <= g.N);
+  // One result as a dot product takes the wave 2 µs (K = 4096, contiguous operands)
+  // to 5 µs (strided).
+  constexpr int kDots = AK && BKC ? 32 : 8;
+  if (nfl > kDots || __any(worst >= 0x7f800000u)) rough = 2;
+  __syncthreads();
+  if (rough == 2) {
+    // The block's tile with the fp32 MFMA: 32 k at a time through LDS as they are,
+    // the next ones loaded under the products.  (k-groups of 16: lane group g holds
+    // the k 4g … 4g + 3 of each.)
+    auto load = [&](int kt) {
+      if (kt + 1 == nk && ktail) {
+        la.template load_all<true>(ktail);
+        lb.template load_all<true>(ktail);
+      } else {
+        la.template load_all<false>(0);
+        lb.template load_all<false>(0);
+      }
+      la.advance();
+      lb.advance();
+    };
+    la.init(g.A, g.lda, m0, g.M, kbeg, tid);
+    lb.init(g.B, g.ldb, n0, g.N, kbeg, tid);
+    load(0);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int kt = 0; kt < nk; ++kt) {
+      char* st = smem + (kt & 1) * STAGE;
+#pragma unroll
+      for (int o = 0; o < NOA; ++o) la.align(o);
+#pragma unroll
+      for (int o = 0; o < NOB; ++o) lb.align(o);
+      la.store_fp32(st);
+      lb.store_fp32(st + BM * 128);
+      __syncthreads();
+      if (kt + 1 < nk) load(kt + 1);
+#pragma unroll
+      for (int q = 0; q < 8; q += 4) {
+        floatx4 a, b[TN];
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          b[j] = *reinterpret_cast<const floatx4*>(st + BM * 128 + fp32_granule(wn * WN + 16 * j + l16, q + g16));
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          a = *reinterpret_cast<const floatx4*>(st + fp32_granule(wm * WM + 16 * i + l16, q + g16));
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = mfma16x16x4(a[e], b[j][e], acc[i][j]);
+        }
+      }
+    }
+    nfl = 0;
+  }
+  if (nfl == 0) {  // the usual way out
+    write_tiles(g, acc, r0, c0, g16, l16, m0 + BM <= g.M && n0 + BN <= g.N);
+    return;
+  }
+  // The masks go to LDS (no wave reads the stages any more) for a loop over strips
+  // of 16 rows.
+  unsigned short* masks = reinterpret_cast<unsigned short*>(smem) + wave * (TM * 64) + lane;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) masks[64 * i] = (unsigned short)fl[i];
+  write_tiles(g, acc, r0, c0, g16, l16, false, [&](int i, int j, int e) { return fl[i] >> (4 * j + e) & 1; });
+#pragma unroll 1
+  for (int i = 0; i < TM; ++i) {
+    unsigned mine = masks[64 * i];
+#pragma unroll 1
+    for (unsigned long long who = __ballot(mine); who; who = __ballot(mine)) {
+      const int at = __ffsll(who) - 1, q = __ffs(__builtin_amdgcn_readlane(mine, at)) - 1;
+      if (lane == at) mine &= mine - 1;
+      const int r = r0 + 16 * i + 4 * (at >> 4) + (q & 3), c = c0 + 16 * (q >> 2) + (at & 15);
+      const float v = fp32_dot<AK, BKC>(g, r, c, kbeg, kend, lane);
+      if (lane == 0) {
+        if (g.split)
+          g.P[((size_t)blockIdx.z * g.M + r) * g.N + c] = v;
+        else
+          apply_epilogue(g.epi, g.C, (size_t)r * g.ldc + c, v);
+      }
+    }
+  }
 }
 
 template <int BM, int BN, int WGM, int WGN>

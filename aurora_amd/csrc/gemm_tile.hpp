@@ -78,10 +78,14 @@ __device__ __forceinline__ void apply_epilogue(const aur::Epilogue& e, float* __
 // Writes a wave's TM×TN grid of 16×16 accumulator tiles (lane holds rows
 // 4·g16 + e, column l16 of each) with the epilogue mode fixed at compile
 // time, so the store loops carry no per-element branch.  MODE −1: split-K
-// partial tile into P[z].  `full`: every row and column is in range.
-template <int MODE, int TM, int TN>
+// partial tile into P[z].  `full`: every row and column is in range, and skip
+// leaves out nothing.
+struct SkipNone {
+  __device__ __forceinline__ bool operator()(int, int, int) const { return false; }
+};
+template <int MODE, int TM, int TN, class Skip>
 __device__ __forceinline__ void write_tile(const GemmArgs& g, const floatx4 (&acc)[TM][TN], int r0, int c0,
-                                           int g16, int l16, bool full) {
+                                           int g16, int l16, bool full, Skip skip) {
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -90,7 +94,7 @@ __device__ __forceinline__ void write_tile(const GemmArgs& g, const floatx4 (&ac
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int row = r0 + i * 16 + 4 * g16 + e;
-        if (!full && (row >= g.M || col >= g.N)) continue;
+        if (!full && (row >= g.M || col >= g.N || skip(i, j, e))) continue;
         const float v = acc[i][j][e];
         if constexpr (MODE < 0) {
           g.P[((size_t)blockIdx.z * g.M + row) * g.N + col] = v;
@@ -108,19 +112,19 @@ __device__ __forceinline__ void write_tile(const GemmArgs& g, const floatx4 (&ac
     }
 }
 
-template <int TM, int TN>
+template <int TM, int TN, class Skip = SkipNone>
 __device__ __forceinline__ void write_tiles(const GemmArgs& g, const floatx4 (&acc)[TM][TN], int r0, int c0,
-                                            int g16, int l16, bool full) {
+                                            int g16, int l16, bool full, Skip skip = Skip()) {
   if (g.split) {
-    write_tile<-1>(g, acc, r0, c0, g16, l16, full);
+    write_tile<-1>(g, acc, r0, c0, g16, l16, full, skip);
     return;
   }
   switch (g.epi.mode) {
-    case aur::EPI_ACCUM: write_tile<aur::EPI_ACCUM>(g, acc, r0, c0, g16, l16, full); break;
-    case aur::EPI_RESID: write_tile<aur::EPI_RESID>(g, acc, r0, c0, g16, l16, full); break;
-    case aur::EPI_GELU: write_tile<aur::EPI_GELU>(g, acc, r0, c0, g16, l16, full); break;
-    case aur::EPI_GELU_BWD: write_tile<aur::EPI_GELU_BWD>(g, acc, r0, c0, g16, l16, full); break;
-    default: write_tile<aur::EPI_STORE>(g, acc, r0, c0, g16, l16, full); break;
+    case aur::EPI_ACCUM: write_tile<aur::EPI_ACCUM>(g, acc, r0, c0, g16, l16, full, skip); break;
+    case aur::EPI_RESID: write_tile<aur::EPI_RESID>(g, acc, r0, c0, g16, l16, full, skip); break;
+    case aur::EPI_GELU: write_tile<aur::EPI_GELU>(g, acc, r0, c0, g16, l16, full, skip); break;
+    case aur::EPI_GELU_BWD: write_tile<aur::EPI_GELU_BWD>(g, acc, r0, c0, g16, l16, full, skip); break;
+    default: write_tile<aur::EPI_STORE>(g, acc, r0, c0, g16, l16, full, skip); break;
   }
 }
 

@@ -18,9 +18,15 @@ __device__ __forceinline__ floatx4 mfma_f16(half8 a, half8 b, floatx4 c) {
 __device__ __forceinline__ float exp_scale(int p) { return __uint_as_float((unsigned)(p + 127) << 23); }
 
 // h = fp16(x·s), l = fp16(x·s − h) of two values.
+__device__ __forceinline__ half2v split_high(float x0, float x1, float s0, float s1) {
+  return __builtin_convertvector(float2v{x0 * s0, x1 * s1}, half2v);
+}
+__device__ __forceinline__ half2v split_low(float x0, float x1, float s0, float s1, half2v h) {
+  return __builtin_convertvector(float2v{__builtin_fmaf(x0, s0, -(float)h[0]), __builtin_fmaf(x1, s1, -(float)h[1])}, half2v);
+}
 __device__ __forceinline__ void split2(float x0, float x1, float s0, float s1, half2v& h, half2v& l) {
-  h = __builtin_convertvector(float2v{x0 * s0, x1 * s1}, half2v);
-  l = __builtin_convertvector(float2v{__builtin_fmaf(x0, s0, -(float)h[0]), __builtin_fmaf(x1, s1, -(float)h[1])}, half2v);
+  h = split_high(x0, x1, s0, s1);
+  l = split_low(x0, x1, s0, s1, h);
 }
 
 // Byte offset of granule q (8 k, 16 bytes) of row r in an LDS plane [ROWS][32]:

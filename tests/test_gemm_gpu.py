@@ -432,10 +432,10 @@ def test_gemm_ex_rejects_short_leading_dimensions(ctx):
 # ---- the split-fp16 kernel (gemm_split.hip), every tile forced
 
 
-def _split_ex(ctx, monkeypatch, cfg, a, b, ak, bk, splits=1):
+def _split_ex(ctx, monkeypatch, cfg, a, b, ak, bk, splits=1, c0=None):
     """op(A)·op(B) of float32 [m, k] and [k, n] arrays through aur_gemm_ex, the
     operands stored with the given orders and a leading dimension one longer
-    than the row (so that no row is 16-byte aligned)."""
+    than the row (so that no row is 16-byte aligned); added to c0 if given."""
     from aurora_amd.gpu import GpuBuffer
 
     def stored(x):
@@ -447,8 +447,9 @@ def _split_ex(ctx, monkeypatch, cfg, a, b, ak, bk, splits=1):
     monkeypatch.setenv("AUR_GEMM_CFG", f"{cfg}:{splits}")
     ab = GpuBuffer.from_slice(ctx, stored(a if ak else a.T))
     bb = GpuBuffer.from_slice(ctx, stored(b.T if bk else b))
-    cb = GpuBuffer.zeros(ctx, m * n)
-    ctx.call("aur_gemm_ex", ak, bk, ab.ptr, (k if ak else m) + 1, bb.ptr, (k if bk else n) + 1, cb.ptr, n, m, n, k, 0)
+    cb = GpuBuffer.zeros(ctx, m * n) if c0 is None else GpuBuffer.from_slice(ctx, c0.ravel())
+    ctx.call("aur_gemm_ex", ak, bk, ab.ptr, (k if ak else m) + 1, bb.ptr, (k if bk else n) + 1, cb.ptr, n, m, n, k,
+             int(c0 is not None))
     out = cb.download().reshape(m, n)
     for x in (ab, bb, cb):
         x.free()
@@ -485,7 +486,7 @@ def test_split_kernel_scales(ctx, monkeypatch, cfg, ak, bk):
     """Rows and columns whose magnitude grows along K by up to 2^60 (their scale
     is lowered while the sum runs), starts with zeros, is tiny (2^-130) or huge
     (2^100): the error stays at 2^-20 of ‖row of A‖·‖column of B‖, element by
-    element (the split's 2^-38 of the largest value is far below it)."""
+    element.  (test_split_kernel_wide_rows bounds it by the products themselves.)"""
     m, n, k = 130, 140, 333
     rng = np.random.default_rng(3)
     a = rng.standard_normal((m, k))
@@ -508,6 +509,67 @@ def test_split_kernel_scales(ctx, monkeypatch, cfg, ak, bk):
         err = np.abs(got - a64 @ b64)
         # below 2^-126 a float itself has an absolute spacing of 2^-149
         assert np.all(err <= 2.0 ** -20 * bound + 2.0 ** -148), (cfg, splits, np.max(err / np.maximum(bound, 1e-300)))
+
+
+def _wide_operands(name, m, n, k):
+    """Finite operands of wide range, [m, k] and [k, n], whose small values matter."""
+    rng = np.random.default_rng(11)
+    a, b, t = rng.standard_normal((m, k)), rng.standard_normal((k, n)), np.arange(k)
+    if name.startswith("outlier"):  # one large value a row, met by zeros
+        a[:, rng.integers(0, k)] = 2.0 ** int(name[8:])
+        b[a[0] == a[0].max()] = 0
+    elif name == "ones":
+        a[:], b[:] = 1, 1
+        a[:, 0], b[0] = 1e10, 0
+    elif name == "late":  # the large value lowers the scale of a sum that was all there is
+        a[:, : k // 2] *= 2.0 ** -100
+        b[k // 2 :] = 0
+    elif name == "octets":  # a large value among every eight
+        a[:, ::8] *= 2.0 ** 24
+        b[::8] = 0
+    elif name == "reciprocal":
+        s = 2.0 ** rng.permutation(np.linspace(-25, 25, k))
+        a, b = a * s, b / s[:, None]
+    elif name == "one-hot":  # single values of a row that happen to be small
+        a[::3, 5] *= 2.0 ** -30
+        b[:] = 0
+        b[t[: min(n, k)], t[: min(n, k)]] = 1
+    elif name == "few":  # a few results of a tile made of small values only
+        a[:, 7] = 2.0 ** -18
+        b[:, 9] = 0
+        b[7, 9] = 3
+        b[:, 40:] = 0
+    elif name == "zeros":  # rows and columns of zeros, and zeros first
+        a[::4], a[1::4, : k // 2], b[:, ::5], b[: k // 2, 1::5] = 0, 0, 0, 0
+        a[2::4, k // 2 :] *= 2.0 ** -40
+    else:  # softmax gradient
+        p = np.exp(6 * a)
+        a = p / p.sum(1, keepdims=True)
+        a[np.arange(m), rng.integers(0, k, m)] -= 1
+    return a.astype(np.float32), b.astype(np.float32)
+
+
+@pytest.mark.parametrize("cfg", SPLIT_TILES)
+@pytest.mark.parametrize("name", ["outlier 8", "outlier 16", "outlier 24", "outlier 60", "ones", "late", "octets",
+                                  "reciprocal", "one-hot", "few", "zeros", "softmax"])
+def test_split_kernel_wide_rows(ctx, monkeypatch, cfg, name):
+    """Values far below the largest of their row or column, where that meets zeros or
+    small values: bound per element, in units of (|A||B|)_ij, that of
+    test_split_kernel_edges, (9 + K/32)·2^-24, and the 2^-21 that a result is let
+    stand at; what is computed again in fp32 rounds once a product, K·2^-24 at most
+    and √K·2^-24 usually.  Below 2e-6 for K = 333 all the same."""
+    m, n, k = 150, 141, 333
+    a, b = _wide_operands(name, m, n, k)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    c0 = (np.random.default_rng(12).standard_normal((m, n)) * np.abs(a64 @ b64)).astype(np.float32)
+    for ak, bk, splits in [(1, 1, 1), (1, 0, 1), (0, 1, 1), (0, 0, 1), (1, 1, 3)]:
+        for start in (None, c0):
+            got = _split_ex(ctx, monkeypatch, cfg, a, b, ak, bk, splits, start).astype(np.float64)
+            want, bound = a64 @ b64, np.abs(a64) @ np.abs(b64)
+            if start is not None:
+                want, bound = want + start, bound + np.abs(start)
+            err = np.abs(got - want)
+            assert np.all(err <= 2e-6 * bound + 2.0 ** -148), (cfg, name, ak, bk, splits, np.max(err / np.maximum(bound, 1e-300)))
 
 
 @pytest.mark.parametrize("cfg", SPLIT_TILES)
