@@ -327,7 +327,14 @@ __global__ void __launch_bounds__(256, 2) mha_fwd_split_kernel(AttnArgs a) {
       all_lo = min(all_lo, (unsigned)in);
       all_hi = min(all_hi, (unsigned)(in >> 32));
     }
-    if (min(all_lo, all_hi) == 0) wide = 1;
+    if (min(all_lo, all_hi) == 0) {  // a row of zeros has nothing to lose
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float m = fmaxf(fabsf(vx[0][i]), fabsf(vx[1][i]));
+        const unsigned long long in = __ballot(m >= thr), some = __ballot(m > 0.f);
+        if (((unsigned)in == 0 && (unsigned)some != 0) || ((in >> 32) == 0 && (some >> 32) != 0)) wide = 1;
+      }
+    }
 #pragma unroll
     for (int i = 0; i < KS; ++i) {
       half8 hh, ll;

@@ -496,6 +496,21 @@ def test_split_forward_matches_float64(ctx, t, h, dh, b):
     assert e < 5e-7, e
 
 
+def test_split_forward_zero_rows_stay(ctx):
+    """Keys of zero V are no reason to compute a block again in fp32: queries before
+    the first of them come out bit by bit as without them."""
+    b, t, h, dh = 16, 300, 6, 64
+    rng = np.random.default_rng(9)
+    q, k, v = (rng.standard_normal((b, t, h, dh)).astype(np.float32) for _ in range(3))
+    v[:, [3, 70, 130, 260]] *= 4  # each tile's largest values stay
+    want, _ = _fwd_bthd(ctx, q, k, v, t, h, dh, b)
+    v[:, [40, 41, 100, 200, 299]] = 0
+    got, _ = _fwd_bthd(ctx, q, k, v, t, h, dh, b)
+    assert np.array_equal(got[:, :40], want[:, :40])
+    o64, _ = causal_attention_f64(*(x.astype(np.float64) for x in (q, k, v)))
+    assert np.linalg.norm(got - o64) / np.linalg.norm(o64) < 5e-7
+
+
 def test_split_forward_non_finite(ctx):
     """Infinities and NaN reach the same outputs as in the fp32 kernel, which a
     single head runs."""
