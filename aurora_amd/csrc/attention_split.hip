@@ -44,6 +44,10 @@ namespace {
 constexpr int QB = 128;             // queries per block
 constexpr float kPScale = 16384.f;  // P ≤ 1 is split at this scale
 
+// The exponent for Q and K: at most 63, so that 2^-(pq + pk) is a normal number also
+// where both are zero (a masked score is an infinity times it).
+__device__ __forceinline__ int score_exp(float m) { return min(tile_exp(m), 63); }
+
 // The 16 queries from q16 of one head again, with the fp32 MFMA and operands
 // straight from memory (see the head of the file).
 template <int DH>
@@ -174,7 +178,7 @@ __global__ void __launch_bounds__(256, 2) mha_fwd_split_kernel(AttnArgs a) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(x[c][e]));
     }
-    pq[qi] = tile_exp(rows4_max(mx));
+    pq[qi] = score_exp(rows4_max(mx));
     const float s = exp_scale(pq[qi]);
 #pragma unroll
     for (int c = 0; c < KS; ++c)
@@ -312,7 +316,7 @@ __global__ void __launch_bounds__(256, 2) mha_fwd_split_kernel(AttnArgs a) {
     __syncthreads();  // the maxima are there, and every wave is done with the previous tile
     mk = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
     mv = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
-    const int pk = tile_exp(mk), pv_new = min(pv, tile_exp(mv));
+    const int pk = score_exp(mk), pv_new = min(pv, tile_exp(mv));
     again |= mk == INFINITY || mv == INFINITY || pk + pq_min < 16;
     const float sk = kr & 1 ? -exp_scale(pk) : exp_scale(pk), sv = exp_scale(pv_new);
     pv = pv_new;

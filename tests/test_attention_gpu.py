@@ -511,6 +511,20 @@ def test_split_forward_zero_rows_stay(ctx):
     assert np.linalg.norm(got - o64) / np.linalg.norm(o64) < 5e-7
 
 
+def test_split_forward_zero_scores_stay(ctx):
+    """Q and K of zero are no reason to compute a block again in fp32: bit by bit the
+    averages that a K of zero beside another Q gives, whose scores are zero too."""
+    b, t, h, dh = 16, 300, 6, 64
+    rng = np.random.default_rng(10)
+    q, v = (rng.standard_normal((b, t, h, dh)).astype(np.float32) for _ in range(2))
+    k = np.zeros_like(q)
+    want, want_lse = _fwd_bthd(ctx, q, k, v, t, h, dh, b)
+    got, lse = _fwd_bthd(ctx, np.zeros_like(q), k, v, t, h, dh, b)
+    assert np.array_equal(got, want) and np.array_equal(lse, want_lse)
+    o64, _ = causal_attention_f64(*(x.astype(np.float64) for x in (q, k, v)))
+    assert np.linalg.norm(got - o64) / np.linalg.norm(o64) < 5e-7
+
+
 def test_split_forward_non_finite(ctx):
     """Infinities and NaN reach the same outputs as in the fp32 kernel, which a
     single head runs."""
