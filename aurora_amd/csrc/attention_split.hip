@@ -11,8 +11,10 @@
 //
 // Scales: Q (times log2(e)/sqrt(d_head)) per query, K per tile, V by a scale
 // that only falls from tile to tile (the running sum is rescaled with the
-// softmax correction), P by 2^14; the scores' factors go into the exp2
-// argument's FMA.
+// softmax correction), P by 2^14 times a power of two per query and tile that
+// brings its largest value there to ½ … 1 (the small P of a later tile may meet
+// larger V: with 2^14 alone the error was 2.8e-5 for V growing by 2^24); the
+// scores' factors go into the exp2 argument's FMA.
 // Odd keys of K and odd columns of V are scaled by the negative (the MFMA
 // truncates downwards: so the error's sign alternates over a row's scores, and
 // over its results).
@@ -20,13 +22,18 @@
 // per wave crossing the barrier that the tile's stage needs anyway.  A tile's
 // V·P products are summed from zero and added to the corrected sum by the VALU.
 // Queries whose result is not finite, and blocks that met an infinity in a tile
-// or values too far apart for its scale (scores beyond 2^12, V rows 2^14 below
-// the tile's largest), are computed again with the fp32 MFMA.
+// or values too far apart for the scales, are computed again with the fp32 MFMA:
+// scores beyond 2^12; among 16 keys of V, 16 or more values (d_head if that is less:
+// as many as a row or a column has) that are not zero but 2^16 or more below the
+// tile's largest; a V that grows by more than 2^60 from the first tile on.  Fewer
+// small values than that keep an absolute error of 2^-40 of the tile's largest.
+// With all blocks computed again B16 H8 T1024 d_head 64 takes 380 µs, against 85
+// and the fp32 MFMA kernel's 150.
 //
 // Per 16×16 scores the MFMAs take 192 cycles (1024 with the fp32 MFMA), the
 // softmax, the split of P and this wave's share of K's and V's about 300 VALU
 // cycles; the sum of the two bounds it (the waves of a SIMD hardly overlap
-// them).  Measured at B16 H8 T1024 d_head 64: 152 → 77 µs against the fp32 MFMA
+// them).  Measured at B16 H8 T1024 d_head 64: 152 → 78 µs against the fp32 MFMA
 // kernel; 16 queries per wave in 8-wave blocks (twice the LDS reads): 93; two
 // LDS stages with one barrier per tile: 78.
 #include "attention.hpp"
@@ -42,7 +49,8 @@ using namespace aursplit;
 namespace {
 
 constexpr int QB = 128;             // queries per block
-constexpr float kPScale = 16384.f;  // P ≤ 1 is split at this scale
+constexpr float kPScale = 16384.f;  // P ≤ 1 is split at this scale and 2^r, r ≤ kPExpMax
+constexpr int kPExpMax = 60;
 
 // The exponent for Q and K: at most 63, so that 2^-(pq + pk) is a normal number also
 // where both are zero (a masked score is an infinity times it).
@@ -118,7 +126,7 @@ __global__ void __launch_bounds__(256, 2) mha_fwd_split_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(1024))) char ks[2 * G::KPLANE];
   __shared__ __attribute__((aligned(1024))) char vs[2 * G::VPLANE];
   __shared__ float red[2][4];  // this tile's largest |K| and |V| of each wave
-  __shared__ int wide;         // a V row far below its tile's largest value was met
+  __shared__ int wide;         // too many values of V far below their tile's largest were met
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 4, l16 = lane & 15;
   const int nqb = (a.T + QB - 1) / QB;
@@ -194,11 +202,13 @@ __global__ void __launch_bounds__(256, 2) mha_fwd_split_kernel(AttnArgs a) {
   const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
   floatx4 acc[2][DT];
   float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};
+  int pr[2] = {0, 0};  // the exponent r of P in the last tile: of the sums too
 #pragma unroll
   for (int qi = 0; qi < 2; ++qi)
 #pragma unroll
     for (int d = 0; d < DT; ++d) acc[qi][d] = zero;
   int pv = 127, pva = 127;  // V's scale so far, and when this wave last added to its sums
+  int pv_top = -127;        // V's scale in the first tile that is not zero
   bool again = false;  // the block met an infinity, or values too far apart for a tile's scale
   // Scores up to about 2^12 keep an absolute error of 2^-24 however small their
   // key is beside the tile's largest; beyond that the fp32 MFMA computes them.
@@ -255,16 +265,18 @@ __global__ void __launch_bounds__(256, 2) mha_fwd_split_kernel(AttnArgs a) {
       for (int j = 1; j < 4; ++j)
         mx = fmaxf(mx, fmaxf(fmaxf(st[qi][j][0], -st[qi][j][1]), fmaxf(st[qi][j][2], -st[qi][j][3])));
       const float c = ldexpf(1.f, -(pq[qi] + pk));
-      const float m_new = fmaxf(m[qi], rows4_max(mx) * c);
+      const float m_tile = rows4_max(mx) * c, m_new = fmaxf(m[qi], m_tile);
       const float alpha = __builtin_amdgcn_exp2f(m[qi] - m_new);
       m[qi] = m_new;
+      const int r = (int)fminf(m_new - m_tile, (float)kPExpMax);
+      const float at = (float)r - m_new;
       float ps = 0.f;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int e = 0; e < 4; e += 2) {
-          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[qi][j][e], c, -m_new));
-          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[qi][j][e + 1], -c, -m_new));
+          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[qi][j][e], c, at));
+          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[qi][j][e + 1], -c, at));
           ps += p0 + p1;
           half2v hh, ll;
           split2(p0, p1, kPScale, kPScale, hh, ll);
@@ -272,8 +284,9 @@ __global__ void __launch_bounds__(256, 2) mha_fwd_split_kernel(AttnArgs a) {
           ph[qi][j >> 1][i] = hh[0], ph[qi][j >> 1][i + 1] = hh[1];
           pl[qi][j >> 1][i] = ll[0], pl[qi][j >> 1][i + 1] = ll[1];
         }
-      l[qi] = l[qi] * alpha + ps;
-      av[qi] = alpha * vcorr;
+      l[qi] = l[qi] * alpha + ps * exp_scale(-r);
+      av[qi] = alpha * vcorr * exp_scale(r - pr[qi]);
+      pr[qi] = r;
     }
     const int nk = DIAG && jd == 0 ? 1 : 2;  // 32-key groups with anything unmasked
 #pragma unroll
@@ -316,28 +329,31 @@ __global__ void __launch_bounds__(256, 2) mha_fwd_split_kernel(AttnArgs a) {
     __syncthreads();  // the maxima are there, and every wave is done with the previous tile
     mk = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
     mv = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
-    const int pk = score_exp(mk), pv_new = min(pv, tile_exp(mv));
+    const int pk = score_exp(mk), pv_new = min(pv, value_exp(mv));
     again |= mk == INFINITY || mv == INFINITY || pk + pq_min < 16;
     const float sk = kr & 1 ? -exp_scale(pk) : exp_scale(pk), sv = exp_scale(pv_new);
     pv = pv_new;
-    // A V row whose largest value is below 2^-14 of the scale's range would
-    // lose relative precision, which a query that sees no larger row would
-    // show.  (Each half of the wave holds one row per i.)
-    const float thr = mv > 0.f ? exp_scale(-pv) : 0.f;
-    unsigned all_lo = ~0u, all_hi = ~0u;
+    // V grown beyond what P's scale can follow
+    if (mv > 0.f) pv_top = max(pv_top, pv);
+    again |= pv_top - pv > kPExpMax;
+    half2v vh[2][4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const unsigned long long in = __ballot(fmaxf(fabsf(vx[0][i]), fabsf(vx[1][i])) >= thr);
-      all_lo = min(all_lo, (unsigned)in);
-      all_hi = min(all_hi, (unsigned)(in >> 32));
-    }
-    if (min(all_lo, all_hi) == 0) {  // a row of zeros has nothing to lose
+    for (int r = 0; r < 2; ++r)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float m = fmaxf(fabsf(vx[0][i]), fabsf(vx[1][i]));
-        const unsigned long long in = __ballot(m >= thr), some = __ballot(m > 0.f);
-        if (((unsigned)in == 0 && (unsigned)some != 0) || ((in >> 32) == 0 && (some >> 32) != 0)) wide = 1;
+      for (int e = 0; e < 8; e += 2) vh[r][e / 2] = split_high(vx[r][e], vx[r][e + 1], r ? -sv : sv, r ? -sv : sv);
+    if (__any((DH == 64 || v_live) && out_of_range(__builtin_elementwise_max(high_range(vh[0]), high_range(vh[1]))))) {
+      int n = 0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) n += count_fine(vx[0][i], sv) + count_fine(vx[1][i], sv);
+      if (n >= G::FINE && k0 + 64 > a.T) {  // the keys past the last one are copies of it
+        n = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const bool in = k0 + 32 * (vg >> 2) + 4 * (vg & 3) + 16 * (i >> 2) + (i & 3) < a.T;
+          n += count_fine(vx[0][i], sv, in) + count_fine(vx[1][i], sv, in);
+        }
       }
+      if (n >= G::FINE) wide = 1;
     }
 #pragma unroll
     for (int i = 0; i < KS; ++i) {
@@ -360,8 +376,7 @@ __global__ void __launch_bounds__(256, 2) mha_fwd_split_kernel(AttnArgs a) {
         const float s = r ? -sv : sv;
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {
-          half2v h2, l2;
-          split2(vx[r][e], vx[r][e + 1], s, s, h2, l2);
+          const half2v h2 = vh[r][e / 2], l2 = split_low(vx[r][e], vx[r][e + 1], s, s, h2);
           hh[e] = h2[0], hh[e + 1] = h2[1];
           ll[e] = l2[0], ll[e + 1] = l2[1];
         }
@@ -392,7 +407,7 @@ __global__ void __launch_bounds__(256, 2) mha_fwd_split_kernel(AttnArgs a) {
     for (int d = 0; d < DT; ++d)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float o = ldexpf(acc[qi][d][e] * (e & 1 ? -inv : inv), -pva);
+        const float o = ldexpf(acc[qi][d][e] * (e & 1 ? -inv : inv), -(pva + pr[qi]));
         acc[qi][d][e] = o;
         bad |= !(o - o == 0.f);
       }

@@ -14,6 +14,10 @@ struct SplitGeo {
   static constexpr int DT = (DH + 15) / 16;  // 16-row tiles of Vᵀ / Oᵀ
   static constexpr int KROW = KS * 64;       // bytes of a K row in LDS
   static constexpr int KPLANE = 64 * KROW, VPLANE = DT * 16 * 128;
+  // Small values among 16 rows of a tile that are one too many: a row of them has
+  // DH, a column 16.  (N(0, 1) values have 0.05 on average, those with
+  // columns 30 times the others' 1.)
+  static constexpr int FINE = DH < 16 ? DH : 16;
 };
 
 // Granule q of row r in rows of 128 bytes: as split_granule, every phase of 16
@@ -30,7 +34,15 @@ __device__ __forceinline__ float wave_max(float v) {
   return rows4_max(v);
 }
 
+// Lanes whose value x is not zero but too small for the scale s.
+__device__ __forceinline__ int count_fine(float x, float s, bool in = true) {
+  return __popcll(__ballot(in & (x != 0.f) & (fabsf(x) * s < kSplitFine)));
+}
+
 // p with max·2^p in [2^13, 2^14).
 __device__ __forceinline__ int tile_exp(float m) { return min(140 - (int)(__float_as_uint(m) >> 23), 127); }
+
+// p with max·2^p in [2^14, 2^15), for values whose small ones are counted.
+__device__ __forceinline__ int value_exp(float m) { return min(141 - (int)(__float_as_uint(m) >> 23), 127); }
 
 }  // namespace aurattn

@@ -71,8 +71,6 @@ typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
 
 // Scale exponent p of a row whose largest magnitude is m (0 when there is none
 // yet), and that of the factor 2^p.
-constexpr float kSplitLimit = 65504.f;  // largest scaled magnitude let through
-constexpr float kSplitFine = 0.25f;     // smallest that keeps its 23 bits
 constexpr float kFineBound = 4096.f;    // |result| ≥ this · (n + m), at the scales: E ≤ 2^-21 of it
 constexpr int kDenseBound = 64;         // n + m ≤ this · (D + D' − 32): E ≤ 2^-21 of that bound
 constexpr int kZeroExp = 127;           // of a row of zeros so far, and of no other (but for values below 2^-111)
@@ -83,21 +81,6 @@ __device__ __forceinline__ int scale_exp(float s) { return (int)((__float_as_uin
 
 // Byte offset of granule q (4 k) of row r in an fp32 tile [ROWS][32].
 __device__ __forceinline__ int fp32_granule(int r, int q) { return r * 128 + ((q ^ r) & 7) * 16; }
-
-// Is any |h| of the octet outside [kSplitFine, kSplitLimit], zero, infinite or NaN?
-// (2h − 2·0x3400 in 16 bits, without the sign, is below 0x9000 for the others.)
-typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ ushort2v high_range(const half2v (&h)[4]) {
-  ushort2v m = {0, 0};
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    ushort2v t;
-    asm("v_pk_mad_u16 %0, %1, 2, %2 op_sel_hi:[1,0,1]" : "=v"(t) : "v"(h[e]), "s"(0x98009800u));
-    m = __builtin_elementwise_max(m, t);
-  }
-  return m;
-}
-__device__ __forceinline__ bool out_of_range(ushort2v t) { return max(t[0], t[1]) >= 0x9000; }
 
 // One operand's share of a thread: NO "octets", each 8 consecutive k of one
 // row (of A, or column of B) in a stage of 32 k.

@@ -496,6 +496,36 @@ def test_split_forward_matches_float64(ctx, t, h, dh, b):
     assert e < 5e-7, e
 
 
+@pytest.mark.parametrize("t,h,dh,b", [(300, 6, 64, 16), (193, 8, 48, 12), (140, 24, 8, 16)])
+@pytest.mark.parametrize("name", ["column -16", "column -24", "column -40", "columns", "rows", "growing 8", "growing 24",
+                                  "growing 40"])
+def test_split_forward_wide_values(ctx, t, h, dh, b, name):
+    """Columns and rows of V far below the others, and values that grow by 2^e from
+    tile to tile while their P falls as much: every column and every row of the result
+    is held to its own norm, to 2e-6 (sums of up to 300 positive weights: the fp32
+    kernel shows 1e-6 and 2e-6) and, as the scores reach e and are rounded to e·2^-24,
+    with their rounding in exp e·2^-22 more."""
+    rng = np.random.default_rng(t + dh)
+    q, k, v = (rng.standard_normal((b, t, h, dh)).astype(np.float32) for _ in range(3))
+    if name.startswith("column "):
+        v[..., 5] *= 2.0 ** int(name[7:])
+    elif name == "columns":
+        v *= (2.0 ** -rng.integers(0, 40, dh)).astype(np.float32)
+    elif name == "rows":
+        v *= (2.0 ** -rng.integers(0, 40, (1, t, 1, 1))).astype(np.float32)
+    else:
+        e = int(name[8:])
+        v[:, 64:] *= 2.0 ** e
+        k[:, 64:], k[:, :64] = 0, 1
+        q[:] = e * np.log(2) / dh ** 0.5  # scores of the first 64 keys: e·log(2) more
+    o, _ = _fwd_bthd(ctx, q, k, v, t, h, dh, b)
+    o64, _ = causal_attention_f64(*(x.astype(np.float64) for x in (q, k, v)))
+    limit = 2e-6 + (int(name[8:]) * 2.0 ** -22 if name.startswith("growing") else 0)
+    for axis in {"columns": [1], "rows": [3]}.get(name, [1, 3]):  # (the others of the two may cancel)
+        e = np.linalg.norm(o - o64, axis=axis) / np.linalg.norm(o64, axis=axis)
+        assert e.max() < limit, (name, axis, e.max())
+
+
 def test_split_forward_zero_rows_stay(ctx):
     """Keys of zero V are no reason to compute a block again in fp32: queries before
     the first of them come out bit by bit as without them."""
