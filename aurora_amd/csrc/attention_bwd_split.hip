@@ -17,9 +17,13 @@
 // added to the fp32 sums by the VALU.
 //
 // A block whose results are not finite, or that met values too far apart for a
-// tile's scale (scores beyond 2^12, a row of Q or dO 2^14 below the tile's largest
-// value, a largest value outside 2^±50), computes its keys again with the fp32
-// MFMA before anything of dK and dV is written.
+// tile's scale, computes its keys again with the fp32 MFMA before anything of dK and
+// dV is written: scores beyond 2^12; among 16 queries of Q or dO, 16 or more values
+// that are not zero but 2^16 or more below the tile's largest (a row or a column has
+// as many); a largest value outside 2^±50.  Fewer small values than that keep an
+// absolute error of 2^-40 of the tile's largest.  With all blocks computed again the
+// backward of B16 H8 T1024 d_head 64 takes 590 µs, against 275 and the fp32 MFMA
+// pass's 392.
 //
 // Per 16×16 scores the MFMAs take 384 cycles (2048 with the fp32 MFMA); the
 // exponentials, the split of P and dS, this wave's share of Q's and dO's and the
@@ -40,9 +44,9 @@ namespace {
 constexpr int KB = 128;  // keys per block
 
 // Largest value of a tile or row outside 2^±50, infinite or not.
-__device__ __forceinline__ bool out_of_range(float m) { return m >= 0x1p50f || (m > 0.f && m < 0x1p-50f); }
-// The scale's exponent for such a value in range (also the sum of two keeps 2^-p normal).
-__device__ __forceinline__ int row_exp(float m) { return max(-37, min(63, tile_exp(m))); }
+__device__ __forceinline__ bool too_far(float m) { return m >= 0x1p50f || (m > 0.f && m < 0x1p-50f); }
+// A scale's exponent for such a value in range (also the sum of two keeps 2^-p normal).
+__device__ __forceinline__ int clamp_exp(int p) { return max(-37, min(63, p)); }
 
 template <int DH>
 struct DkvSplitLds {
@@ -77,8 +81,8 @@ __device__ __forceinline__ int split_row(const float* row, float mul, int g, hal
     for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(x[c][e]));
   }
   mx = rows4_max(mx);
-  far |= out_of_range(mx);
-  const int p = row_exp(mx);
+  far |= too_far(mx);
+  const int p = clamp_exp(tile_exp(mx));
   const float s = exp_scale(p);
 #pragma unroll
   for (int c = 0; c < KS; ++c)
@@ -135,19 +139,17 @@ __global__ void __launch_bounds__(256, 2) mha_bwd_dkv_split_kernel(AttnArgs a) {
       r_D = a.D[stat + q];
     }
   };
-  // The thread's values to both layouts of one tensor; true if a row that is not
-  // zero lies too far below the tile's scale.  (A half wave holds one row per i.)
-  auto lay_down = [&](const float2v* x, int p, char* rows, char* cols) {
-    const float s = exp_scale(p), thr = exp_scale(-p);
-    unsigned in_lo = ~0u, in_hi = ~0u;
+  // The thread's values to both layouts of one tensor; true if too many of the wave's
+  // 16 queries are too small for the tile's scale (SplitGeo::FINE).
+  auto lay_down = [&](const float2v* x, int q0, int p, char* rows, char* cols) {
+    const float s = exp_scale(p);
     half8 th[2], tl[2];
+    half2v all[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const unsigned long long in = __ballot(fmaxf(fabsf(x[i][0]), fabsf(x[i][1])) >= thr);
-      in_lo = min(in_lo, (unsigned)in);
-      in_hi = min(in_hi, (unsigned)(in >> 32));
       half2v hh, ll;
       split2(x[i][0], x[i][1], i & 1 ? -s : s, i & 1 ? s : -s, hh, ll);
+      all[i] = hh;
       th[0][i] = hh[0], th[1][i] = hh[1];
       tl[0][i] = ll[0], tl[1][i] = ll[1];
       if (KS == 2 || 2 * vp < KS * 32) {
@@ -164,16 +166,15 @@ __global__ void __launch_bounds__(256, 2) mha_bwd_dkv_split_kernel(AttnArgs a) {
         *reinterpret_cast<half8*>(c + G::VPLANE) = tl[r];
       }
     }
-    bool wide = false;
-    if (min(in_lo, in_hi) == 0) {
+    int n = 0;
+    if (__any((DH == 64 || live) && out_of_range(high_range(all)))) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const float m = fmaxf(fabsf(x[i][0]), fabsf(x[i][1]));
-        const unsigned long long in = __ballot(m >= thr), some = __ballot(m > 0.f);
-        wide |= ((unsigned)in == 0 && (unsigned)some != 0) || ((in >> 32) == 0 && (some >> 32) != 0);
+        const bool in = q0 + r0 + 16 * (i >> 2) + (i & 3) < a.T;  // the others are copies of the last
+        n += count_fine(x[i][0], s, in) + count_fine(x[i][1], s, in);
       }
     }
-    return wide;
+    return n >= G::FINE;
   };
 
   // K and V fragments: key column l16 of tile ki, octet g of step c.
@@ -310,12 +311,12 @@ __global__ void __launch_bounds__(256, 2) mha_bwd_dkv_split_kernel(AttnArgs a) {
     __syncthreads();  // the maxima are there, and every wave is done with the previous tile
     mq = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
     mo = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
-    const int pq = row_exp(mq), po = row_exp(mo);
+    const int pq = clamp_exp(value_exp(mq)), po = clamp_exp(value_exp(mo));
     // Scores up to about 2^12 keep an absolute error of 2^-24 however small their
     // query is beside the tile's largest.
-    far |= out_of_range(mq) || out_of_range(mo) || pq + pk_min < 16;
-    far |= lay_down(qx, pq, lds.s.q, lds.s.qt);
-    far |= lay_down(ox, po, lds.s.o, lds.s.ot);
+    far |= too_far(mq) || too_far(mo) || pq + pk_min < 17;
+    far |= lay_down(qx, q0, pq, lds.s.q, lds.s.qt);
+    far |= lay_down(ox, q0, po, lds.s.o, lds.s.ot);
     if (tid < TQ) {  // queries past T: P = exp2(S - inf) = 0
       lds.s.lse[tid] = q0 + tid < a.T ? r_lse * LOG2E : INFINITY;
       lds.s.D[tid] = q0 + tid < a.T ? r_D : 0.f;

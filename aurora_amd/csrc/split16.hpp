@@ -32,13 +32,14 @@ __device__ __forceinline__ void split2(float x0, float x1, float s0, float s1, h
 constexpr float kSplitLimit = 65504.f;  // largest scaled magnitude let through
 constexpr float kSplitFine = 0.25f;     // smallest that keeps its 23 bits
 
-// Is any |h| of four pairs outside [kSplitFine, kSplitLimit], zero, infinite or NaN?
+// Is any |h| of N pairs outside [kSplitFine, kSplitLimit], zero, infinite or NaN?
 // (2h − 2·0x3400 in 16 bits, without the sign, is below 0x9000 for the others.)
 typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ ushort2v high_range(const half2v (&h)[4]) {
+template <int N>
+__device__ __forceinline__ ushort2v high_range(const half2v (&h)[N]) {
   ushort2v m = {0, 0};
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
+  for (int e = 0; e < N; ++e) {
     ushort2v t;
     asm("v_pk_mad_u16 %0, %1, 2, %2 op_sel_hi:[1,0,1]" : "=v"(t) : "v"(h[e]), "s"(0x98009800u));
     m = __builtin_elementwise_max(m, t);

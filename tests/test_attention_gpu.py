@@ -614,6 +614,32 @@ def test_split_backward_matches_float64(ctx, t, h, dh, b):
             assert e.max() < 2.0 ** -14, (np.unravel_index(e.argmax(), e.shape), e.max())
 
 
+@pytest.mark.parametrize("t,h,dh,b", [(300, 10, 64, 16), (193, 14, 48, 16)])
+@pytest.mark.parametrize("name", ["column -16", "column -24", "column -40", "columns", "rows"])
+def test_split_backward_wide_values(ctx, t, h, dh, b, name):
+    """Columns and rows of dO and Q far below the others: every column of dK and dV
+    (a sum with positive weights over dO) is held to its own norm, 5e-6, and every
+    row of dV to 1e-5; the fp32 pass shows 2e-6."""
+    rng = np.random.default_rng(t + dh)
+    q, k, v, do = (rng.standard_normal((b, t, h, dh)).astype(np.float32) for _ in range(4))
+    for x, at in ((q, 7), (do, 5)):
+        if name.startswith("column "):
+            x[..., at] *= 2.0 ** int(name[7:])
+        elif name == "columns":
+            x *= (2.0 ** -rng.integers(0, 30, dh)).astype(np.float32)
+        else:
+            x *= (2.0 ** -rng.integers(0, 30, (1, t, 1, 1))).astype(np.float32)
+    o, lse = _fwd_bthd(ctx, q, k, v, t, h, dh, b)
+    _, dk, dv = _bwd(ctx, *(x.ravel() for x in (q, k, v, o, lse, do)), b, t, h, dh)
+    _, dk64, dv64 = causal_attention_grad_f64(*(x.astype(np.float64) for x in (q, k, v, do)))
+    for what, got, want, axis, limit in (("dk", dk, dk64, 1, 5e-6), ("dv", dv, dv64, 1, 5e-6), ("dv", dv, dv64, 3, 1e-5)):
+        got = got.reshape(b, t, h, dh)
+        if name == "rows" and axis == 1 or name == "columns" and axis == 3:
+            continue  # these may cancel
+        e = np.linalg.norm(got - want, axis=axis) / np.linalg.norm(want, axis=axis)
+        assert e.max() < limit, (name, what, axis, e.max())
+
+
 def test_split_backward_non_finite(ctx):
     """Infinities and NaN reach the same gradients as in the fp32 kernel, which a
     single head runs; gradients are added to what is there."""
