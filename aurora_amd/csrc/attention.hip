@@ -626,26 +626,26 @@ unsigned pad_grid(size_t n) { return (unsigned)std::min<size_t>((n + 255) / 256,
 // 82, 40 134 → 78, 32 86 → 56, 16 52 → 46).  With about one block per CU both
 // kernels wait on one block's chain of tiles, which its 128-query blocks do not
 // shorten: it starts to win at 1.25 64-query blocks per CU (16×4 heads of T 300:
-// 17.2 → 16.8 µs; 6×4 of T 333: 16.6 → 18.5), later at narrow heads, whose fp32
+// 17.2 → 16.8 µs; 6×4 of T 333: 16.6 → 18.5), at 4 with narrow heads, whose fp32
 // products are short (9×11 heads of 16, T 192: 6.1 → 9.1), and not at one or two
 // tiles (T 128: 10.3 → 10.8 µs at 16×12 heads of 64).
-bool fwd_takes_split(uint32_t b, uint32_t t, uint32_t n_head, uint32_t d_head) {
-  const size_t blocks = (size_t)b * n_head * ((t + TQ - 1) / TQ);
-  return t > 2 * TQ && blocks >= (d_head <= 16 ? 1024 : 320);
+bool fwd_takes_split(const aur_ctx* ctx, uint32_t b, uint32_t t, uint32_t n_head, uint32_t d_head) {
+  const size_t blocks = (size_t)b * n_head * ((t + TQ - 1) / TQ), cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  return t > 2 * TQ && 4 * blocks >= (d_head <= 16 ? 16 : 5) * cus;
 }
 
 // The split-fp16 dK/dV pass (attention_bwd_split.hip), by the whole backward's
 // time: B16 H8 T1024, d_head 64 392 → 274 µs, 56 437 → 293, 40 333 → 252, 32 234
 // → 195, 24 246 → 200, but 16 151 → 166 (its fp32 products are short).  Its
-// 128-key blocks need enough of them: d_head ≥ 40 breaks even at 512 64-key tiles
-// (4×8 heads of T 1024: 156 → 151 µs, 16×8 of T 256: 52.5 → 53.7, 16×6 of T 300:
-// 53 → 56) and gains from 640 on (16×8 of T 384: 85 → 76), narrower heads from
-// 1024 and T > 256 (8×8 of T 1024, d_head 32: 140 → 125; at 512: 98 → 114; 32×32 of
+// 128-key blocks need enough of them: d_head ≥ 40 breaks even at two 64-key tiles
+// per CU (4×8 heads of T 1024: 156 → 151 µs, 16×8 of T 256: 52.5 → 53.7, 16×6 of T 300:
+// 53 → 56) and gains from 2.5 on (16×8 of T 384: 85 → 76), narrower heads from
+// 4 and T > 256 (8×8 of T 1024, d_head 32: 140 → 125; at 2: 98 → 114; 32×32 of
 // T 160, d_head 24: 120 → 125).  One or two tiles stay in fp32 (16×12 heads of 64,
 // T 128: 34 → 37 µs; three: 32×16 heads of 64, T 129: 92 → 82).
-bool bwd_takes_split(uint32_t b, uint32_t t, uint32_t n_head, uint32_t d_head) {
-  const size_t tiles = (size_t)b * n_head * ((t + TQ - 1) / TQ);
-  return d_head >= 40 ? t > 2 * TQ && tiles >= 640 : d_head > 16 && t > 4 * TQ && tiles >= 1024;
+bool bwd_takes_split(const aur_ctx* ctx, uint32_t b, uint32_t t, uint32_t n_head, uint32_t d_head) {
+  const size_t tiles = (size_t)b * n_head * ((t + TQ - 1) / TQ), cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  return d_head >= 40 ? t > 2 * TQ && 2 * tiles >= 5 * cus : d_head > 16 && t > 4 * TQ && tiles >= 4 * cus;
 }
 
 template <int DH>
@@ -661,13 +661,14 @@ void launch_fwd(const AttnArgs& a, int b, hipStream_t st) {
 }
 
 template <int DH>
-void launch_bwd(const AttnArgs& a, int b, hipStream_t st) {
+void launch_bwd(const aur_ctx* ctx, const AttnArgs& a, int b) {
+  const hipStream_t st = ctx->stream;
   constexpr int RPB = 256 / pow2_at_least(DH / 4);  // rows per block of mha_bwd_rowdot_kernel
   const size_t rows = (size_t)b * a.T * a.H;
   hipLaunchKernelGGL(mha_bwd_rowdot_kernel<DH>, dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256),
                      0, st, a, b);
   dim3 grid(a.H, b, (a.T + TQ - 1) / TQ);
-  if (bwd_takes_split((uint32_t)b, (uint32_t)a.T, (uint32_t)a.H, DH))
+  if (bwd_takes_split(ctx, (uint32_t)b, (uint32_t)a.T, (uint32_t)a.H, DH))
     bwd_dkv_split(a, b, DH, st);
   else if (std::getenv("AUR_ATTN_DKV_NS2") == nullptr)
     hipLaunchKernelGGL((mha_bwd_dkv_kernel<DH, 1>), grid, dim3(256), 0, st, a);  // also stores dS, as the split one
@@ -746,14 +747,14 @@ static int mha_bwd_impl(aur_ctx* ctx, int overwrite, bool ws_tiled, const float*
   a.T = (int)t; a.H = (int)n_head;
   a.scale = 1.0f / sqrtf((float)(scale_dh ? scale_dh : d_head));
   switch (d_head) {
-    case 8: launch_bwd<8>(a, (int)b, ctx->stream); break;
-    case 16: launch_bwd<16>(a, (int)b, ctx->stream); break;
-    case 24: launch_bwd<24>(a, (int)b, ctx->stream); break;
-    case 32: launch_bwd<32>(a, (int)b, ctx->stream); break;
-    case 40: launch_bwd<40>(a, (int)b, ctx->stream); break;
-    case 48: launch_bwd<48>(a, (int)b, ctx->stream); break;
-    case 56: launch_bwd<56>(a, (int)b, ctx->stream); break;
-    default: launch_bwd<64>(a, (int)b, ctx->stream); break;
+    case 8: launch_bwd<8>(ctx, a, (int)b); break;
+    case 16: launch_bwd<16>(ctx, a, (int)b); break;
+    case 24: launch_bwd<24>(ctx, a, (int)b); break;
+    case 32: launch_bwd<32>(ctx, a, (int)b); break;
+    case 40: launch_bwd<40>(ctx, a, (int)b); break;
+    case 48: launch_bwd<48>(ctx, a, (int)b); break;
+    case 56: launch_bwd<56>(ctx, a, (int)b); break;
+    default: launch_bwd<64>(ctx, a, (int)b); break;
   }
   AUR_LAUNCH_CHECK(ctx, "mha_bwd kernels");
   return 0;
@@ -796,7 +797,7 @@ int aur_mha_fwd_ex(aur_ctx* ctx, const float* q, const float* k, const float* v,
   a.ld_qkv = (int)ld_qkv; a.ld_o = (int)ld_out;
   a.T = (int)t; a.H = (int)n_head;
   a.scale = 1.0f / sqrtf((float)scale_dh);
-  if (fwd_takes_split(b, t, n_head, d_head))
+  if (fwd_takes_split(ctx, b, t, n_head, d_head))
     fwd_split(a, (int)b, (int)d_head, ctx->stream);
   else
   switch (d_head) {
