@@ -198,6 +198,31 @@ def test_small_tiles_ragged_shapes(ctx, monkeypatch, cfg):
     assert cw < TOL_GEMM and fr < TOL_GEMM, ("outer", cfg, cw, fr)
 
 
+@pytest.mark.parametrize("cfg", ["128x128:1", "128x64:1", "64x64:1", "64x64:4", "64x32:1", "32x32:1"])
+@pytest.mark.parametrize("m,k,n,staged", [(512, 2048, 384, True), (257, 1000, 129, False), (130, 33, 70, False),
+                                          (389, 517, 450, False), (96, 700, 611, False)])
+def test_fp32_tiles_staged_and_ragged(ctx, monkeypatch, cfg, m, k, n, staged):
+    """The register-staged fp32 kernel at every tile: on whole tiles (the override
+    that keeps the direct-load kernel away) and on ragged shapes, which the plan
+    otherwise gives to the split-fp16 kernel.  All three forms against float64."""
+    monkeypatch.setenv("AUR_GEMM_CFG", cfg)
+    if staged:
+        monkeypatch.setenv("AUR_GEMM_STAGED", "1")
+    rng = np.random.default_rng(7200 + m + k + n)
+    a = _u(rng, m * k)
+    b_nn, b_nt = _u(rng, k * n), _u(rng, n * k)
+    a64 = a.reshape(m, k).astype(np.float64)
+    cw, fr = _gates(_nn(ctx, a, b_nn, m, n, k), a64, b_nn.reshape(k, n).astype(np.float64))
+    assert cw < TOL_GEMM and fr < TOL_GEMM, ("nn", cfg, cw, fr)
+    cw, fr = _gates(_nt(ctx, a, b_nt, m, n, k), a64, b_nt.reshape(n, k).T.astype(np.float64))
+    assert cw < TOL_GEMM and fr < TOL_GEMM, ("nt", cfg, cw, fr)
+    x, dy, dest = _u(rng, k * n), _u(rng, k * m), _u(rng, m * n)
+    got = _outer(ctx, x, dy, dest, m, n, k)
+    cw, fr = _gates(got, dy.reshape(k, m).T.astype(np.float64), x.reshape(k, n).astype(np.float64),
+                    dest.reshape(m, n))
+    assert cw < TOL_GEMM and fr < TOL_GEMM, ("outer", cfg, cw, fr)
+
+
 @pytest.mark.parametrize("m,k,n", [(32, 1024, 3072), (32, 1024, 1024), (32, 4096, 1024),
                                    (32, 1024, 8192), (1, 36, 130), (17, 4100, 100), (64, 256, 64),
                                    (48, 2048, 200)])
@@ -471,13 +496,27 @@ def test_split_kernel_edges(ctx, monkeypatch, cfg, ak, bk):
     bm, bn = (int(x) for x in cfg[1:].split("x"))
     rng = np.random.default_rng(1000 * ak + 10 * bk + bm)
     for m, n, k in [(bm - 1, bn + 1, 32), (bm, bn, 64), (bm + 1, bn - 1, 33), (65, 3, 127), (2, 65, 96),
-                    (66, 67, 200), (bm + 63, 2 * bn, 31)]:
-        k = max(k, 64) if k < 32 else k
+                    (66, 67, 200), (bm + 63, 2 * bn, 31), (33, bn + 5, 1)]:
         a = rng.standard_normal((m, k)).astype(np.float32)
         b = rng.standard_normal((k, n)).astype(np.float32)
         got = _split_ex(ctx, monkeypatch, cfg, a, b, ak, bk)
         cw, fr = _gates(got, a.astype(np.float64), b.astype(np.float64))
         assert cw < 1e-6 and fr < 4e-7, (cfg, ak, bk, m, n, k, cw, fr)
+
+
+@pytest.mark.parametrize("cfg", SPLIT_TILES)
+@pytest.mark.parametrize("ak,bk", [(1, 1), (1, 0), (0, 1), (0, 0)])
+def test_split_kernel_short_last_range(ctx, monkeypatch, cfg, ak, bk):
+    """K ranges whose last one has less than one stage of 32 k: 1121 in 8 ranges of
+    160 leaves 1, 300 in 4 of 96 leaves 12.  Bound as in test_split_kernel_edges:
+    (9 + 160/32)·2^-24 a range, and one rounding for each of the ranges added."""
+    rng = np.random.default_rng(2000 + 10 * ak + bk)
+    for m, n, k, splits in [(70, 131, 1121, 8), (70, 131, 300, 4)]:
+        a = rng.standard_normal((m, k)).astype(np.float32)
+        b = rng.standard_normal((k, n)).astype(np.float32)
+        got = _split_ex(ctx, monkeypatch, cfg, a, b, ak, bk, splits)
+        cw, fr = _gates(got, a.astype(np.float64), b.astype(np.float64))
+        assert cw < 1.4e-6 and fr < 4e-7, (cfg, ak, bk, k, cw, fr)
 
 
 @pytest.mark.parametrize("cfg", SPLIT_TILES)
