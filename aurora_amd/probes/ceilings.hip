@@ -1,6 +1,7 @@
 // Ceiling probes for the roofline figures the bench reports: what the GPU
 // under test sustains for
-//   * fp32 MFMA issue with every operand in registers (no memory traffic),
+//   * fp32 and fp16 MFMA issue with every operand in registers (no memory
+//     traffic; the fp16 operands have random bits, as power sets its clock),
 //   * a streaming read of a buffer far larger than the caches (the best of
 //     a few load depths and grid sizes),
 //   * an empty kernel replayed from a HIP graph (the fixed cost every
@@ -51,6 +52,37 @@ __global__ void __launch_bounds__(256) mfma_f32_peak_kernel(int iters, float* si
   sink[(size_t)blockIdx.x * blockDim.x + threadIdx.x] = s;
 }
 
+// v_mfma_f32_16x16x32_f16 (16384 FLOP), the form of the split-fp16 kernels.  The
+// operands' values lie in ±[1, 2) with random mantissas and signs.
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+__global__ void __launch_bounds__(256) mfma_f16_peak_kernel(int iters, float* sink) {
+  unsigned s = (blockIdx.x * 256u + threadIdx.x) * 2654435761u + 12345u;
+  half8 a[2], b[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      s = s * 1664525u + 1013904223u;
+      a[i][e] = __builtin_bit_cast(_Float16, (unsigned short)(0x3c00u | (s >> 22) | (s >> 16 & 0x8000u)));
+      s = s * 1664525u + 1013904223u;
+      b[i][e] = __builtin_bit_cast(_Float16, (unsigned short)(0x3c00u | (s >> 22) | (s >> 16 & 0x8000u)));
+    }
+  floatx4 acc[kChains];
+#pragma unroll
+  for (int j = 0; j < kChains; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < iters; ++i) {
+#pragma unroll
+    for (int r = 0; r < 4 * kChains; ++r)
+      acc[r % kChains] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[r & 1], b[r >> 1 & 1], acc[r % kChains], 0, 0, 0);
+  }
+  float v = 0.f;
+#pragma unroll
+  for (int j = 0; j < kChains; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v += acc[j][e];
+  sink[(size_t)blockIdx.x * blockDim.x + threadIdx.x] = v;
+}
+
 // Grid-stride read: lane i reads float4 i, i + S, i + 2S, … (S = all lanes
 // of the grid), U loads in flight per lane per step.
 template <int U, bool NT>
@@ -96,6 +128,15 @@ double ceil_mfma_f32_32x32_flop(int blocks, int iters) {
 int ceil_mfma_f32_32x32(void* stream, int blocks, int iters, float* sink) {
   if (blocks <= 0 || iters <= 0 || !sink) return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL(mfma_f32_peak_kernel<true>, dim3(blocks), dim3(256), 0, (hipStream_t)stream, iters, sink);
+  return (int)hipGetLastError();
+}
+
+// The same with v_mfma_f32_16x16x32_f16: blocks · 4 · iters · 4 · chains · 2·16·16·32 FLOP.
+double ceil_mfma_f16_flop(int blocks, int iters) { return (double)blocks * 4.0 * iters * 4 * kChains * 16384.0; }
+
+int ceil_mfma_f16(void* stream, int blocks, int iters, float* sink) {
+  if (blocks <= 0 || iters <= 0 || !sink) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(mfma_f16_peak_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, iters, sink);
   return (int)hipGetLastError();
 }
 

@@ -27,15 +27,17 @@ import time
 
 import numpy as np
 
-PEAK_FP32_MFMA = 157.3  # TFLOP/s, MI355X dense fp32 matrix
+PEAK_FP32_MFMA = 157.3  # TFLOP/s, MI355X dense fp32 matrix; "pct_peak" is in units of it, and can pass 100:
+                        # large products run on the fp16 unit, three fp16 products for each fp32 one
+PEAK_FP16_MFMA = 2500.0  # TFLOP/s, dense fp16 matrix
 PEAK_HBM = 8000.0       # GB/s
 
 CLOCK_RAMP_S = 0.25     # untimed sustained work before a timed GEMM region
 COPY_MIB = 256          # calibration copy of the --only traffic leg
 # HBM bytes per head-GEMM launch from the two counter passes of
-# profiles/gemm_head_nt_8192x8192x512_traffic.md: FETCH_SIZE 156261.9 KiB × 2.000
-# + WRITE_SIZE 262144.4 KiB × 1.000 (factors from the 256 MiB copy).
-HEAD_TRAFFIC_BYTES = (156261.9 * 2.000 + 262144.4 * 1.000) * 1024
+# profiles/gemm_head_nt_8192x8192x512_traffic.md: FETCH_SIZE 98799.8 KiB × 2.000
+# + WRITE_SIZE 307904.3 KiB × 1.000 (factors from the 256 MiB copy).
+HEAD_TRAFFIC_BYTES = (98799.8 * 2.000 + 307904.3 * 1.000) * 1024
 SWEEP_KN = [(512, 1536), (512, 512), (512, 2048), (2048, 512)]
 M = 8192
 
@@ -182,8 +184,8 @@ def time_region(ctx, fn, steps: int) -> float:
 
 def bench_ceilings(ctx, cus: int) -> dict:
     """What this GPU sustains, measured with the probes of
-    aurora_amd/probes/ceilings.hip on the library's stream: fp32 MFMA with
-    register operands (2 blocks of 4 waves per CU, 8 independent chains per
+    aurora_amd/probes/ceilings.hip on the library's stream: fp32 and fp16 MFMA
+    with register operands (2 blocks of 4 waves per CU, 8 independent chains per
     wave), a streaming read of 2 GiB (the best of 2-16 blocks per CU with 4
     or 8 float4 loads in flight per lane), and an empty kernel replayed from a HIP graph (per
     launch, over 100 captured launches).  The roofline fractions keep the
@@ -202,6 +204,9 @@ def bench_ceilings(ctx, cus: int) -> dict:
     lib.ceil_mfma_f32_32x32_flop.restype = C.c_double
     lib.ceil_mfma_f32_32x32_flop.argtypes = [C.c_int, C.c_int]
     lib.ceil_mfma_f32_32x32.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_void_p]
+    lib.ceil_mfma_f16_flop.restype = C.c_double
+    lib.ceil_mfma_f16_flop.argtypes = [C.c_int, C.c_int]
+    lib.ceil_mfma_f16.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_void_p]
     lib.ceil_stream_read.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, C.c_int, C.c_void_p]
     lib.ceil_graph_create.argtypes = [C.c_void_p, C.c_int, C.POINTER(C.c_void_p)]
     lib.ceil_graph_reads_create.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, C.c_int, C.c_int,
@@ -226,6 +231,9 @@ def bench_ceilings(ctx, cus: int) -> dict:
     ms32 = time_region(ctx, lambda: ok(lib.ceil_mfma_f32_32x32(stream, mfma_blocks, iters // 2, sink.ptr),
                                         "ceil_mfma_f32_32x32"), 5)
     mfma32_tf = lib.ceil_mfma_f32_32x32_flop(mfma_blocks, iters // 2) / (ms32 * 1e-3) / 1e12
+    # fp16 with fp32 sums, a launch as long again
+    ms16 = time_region(ctx, lambda: ok(lib.ceil_mfma_f16(stream, mfma_blocks, 4 * iters, sink.ptr), "ceil_mfma_f16"), 5)
+    mfma16_tf = lib.ceil_mfma_f16_flop(mfma_blocks, 4 * iters) / (ms16 * 1e-3) / 1e12
 
     nbytes = 2 << 30
     src = GpuBuffer.zeros(ctx, nbytes // 4)
@@ -278,18 +286,19 @@ def bench_ceilings(ctx, cus: int) -> dict:
     big.free()
     sink.free()
     out = {"mfma_fp32_tflops": round(mfma_tf, 1), "mfma_fp32_frac_of_peak": round(mfma_tf / PEAK_FP32_MFMA, 3),
-           "mfma_fp32_32x32x2_tflops": round(mfma32_tf, 1),
+           "mfma_fp32_32x32x2_tflops": round(mfma32_tf, 1), "mfma_fp16_tflops": round(mfma16_tf, 1),
            "hbm_read_gbs": round(read_gbs, 1), "hbm_read_frac_of_peak": round(read_gbs / PEAK_HBM, 3),
            "hbm_read_best": best, "hbm_read_all_gbs": {k: round(v, 1) for k, v in reads.items()},
            "graph_empty_kernel_us": round(ms_g * 1e3 / n_launch, 2),
            "graph_reads": small_reads,
-           "probes": "register-operand fp32 MFMA (16x16x4, and 32x32x2), 2 GiB streaming read, "
+           "probes": "register-operand fp32 MFMA (16x16x4, and 32x32x2) and fp16 MFMA (16x16x32, random operands), 2 GiB streaming read, "
                      "empty kernel in a HIP graph, 4-16 MiB reads replayed from a HIP graph (cold / warm)"}
     log(f"[bench] ceilings {out}")
     return out
 
 
-PLANNER_TILES = ["256x128", "128x128", "128x64", "64x64", "64x32", "32x32"]
+PLANNER_TILES = ["256x128", "128x128", "128x64", "64x64", "64x32", "32x32",  # fp32 kernels
+                 "h256x256", "h256x128", "h128x128", "h64x64"]  # split-fp16 kernel
 PLANNER_SPLITS = [1, 2, 4, 8, 16]
 
 
@@ -313,10 +322,11 @@ def planner_shapes(which: str) -> list[tuple[str, int, int, int]]:
 
 
 def bench_planner(ctx, steps: int, which: str) -> None:
-    """The GEMM launch-plan sweep the planner constants in gemm.hip
-    (choose_plan) are fitted to: every forced tile / split-K configuration
-    (AUR_GEMM_CFG="BMxBN:splits", which the library reads on every call) of
-    each shape, next to the planner's own pick.  One line per (form, shape)
+    """The GEMM launch-plan sweep: every forced tile / split-K configuration
+    (AUR_GEMM_CFG="[h]BMxBN:splits", which the library reads on every call) of
+    each shape, next to the planner's own pick.  The constants of choose_plan
+    (gemm.hip) are fitted to such times, those of the split-fp16 tiles at odd
+    and smaller shapes too.  One line per (form, shape)
     on stdout: "form MxNxK: auto=<TFLOP/s> cfg=<TFLOP/s> ..."; inputs are
     seeded U(-1,1) fp32 in HBM."""
     from aurora_amd.gpu import GpuBuffer
@@ -879,6 +889,8 @@ def main() -> int:
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "fp32",
+        "arithmetic": "fp32 operands, sums and results; large products split each operand value into two fp16 "
+                      "numbers (23 of its 24 bits) and sum three fp16 products in fp32",
         "data": "synthetic (seeded U(-1,1) operands resident in HBM)",
         "config": {"workload": "BASELINE config 1: fp32 GEMM sweep, M=8192, NN+NT for "
                                "(K,N) in {(512,1536),(512,512),(512,2048),(2048,512)}, tied head "
@@ -892,10 +904,12 @@ def main() -> int:
         "train": train,
         "decode": decode,
         "ceilings": ceilings,
-        "roofline": {"bound": "mfma", "kernel": "gemm_f16x3<256,256> (tied head, NT 8192x8192x512; peak: the fp32 MFMA's; "
-                               "traffic: measured with the fp32 MFMA kernel)",
-                     "achieved": round(head_tf, 3), "peak": PEAK_FP32_MFMA, "unit": "TFLOP/s",
-                     "frac": round(head_tf / PEAK_FP32_MFMA, 4), "traffic": round(HEAD_TRAFFIC_BYTES),
+        "roofline": {"bound": "mfma", "kernel": "gemm_f16x3<256,256> (tied head, NT 8192x8192x512; peak: the published dense "
+                               "fp16 rate over the three fp16 products of each fp32 one)",
+                     "achieved": round(head_tf, 3), "peak": round(PEAK_FP16_MFMA / 3, 1), "unit": "TFLOP/s",
+                     "frac": round(3 * head_tf / PEAK_FP16_MFMA, 4),
+                     "frac_of_measured": round(3 * head_tf / ceilings["mfma_fp16_tflops"], 4),
+                     "traffic": round(HEAD_TRAFFIC_BYTES),
                      "traffic_unit": "bytes per launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, copy-calibrated)",
                      "algorithmic_bytes": 4 * (2 * 8192 * 512 + 8192 * 8192)},
         "cpu_baseline": cpu,

@@ -90,6 +90,7 @@ def test_ceiling_probe_library_loads():
 
     lib = C.CDLL(str(PROBE_LIB))
     for name in ("ceil_mfma_f32", "ceil_mfma_f32_flop", "ceil_mfma_f32_32x32", "ceil_mfma_f32_32x32_flop",
+                 "ceil_mfma_f16", "ceil_mfma_f16_flop",
                  "ceil_stream_read", "ceil_graph_create", "ceil_graph_launch", "ceil_graph_destroy"):
         assert hasattr(lib, name), name
     lib.ceil_mfma_f32_flop.restype = C.c_double
