@@ -19,7 +19,7 @@
 // A block whose results are not finite, or that met values too far apart for a
 // tile's scale, computes its keys again with the fp32 MFMA before anything of dK and
 // dV is written: scores beyond 2^12; among 16 queries of Q or dO, 16 or more values
-// that are not zero but 2^16 or more below the tile's largest (a row or a column has
+// that are not zero but 2^18 or more below the tile's largest (a row or a column has
 // as many); a largest value outside 2^±50.  Fewer small values than that keep an
 // absolute error of 2^-40 of the tile's largest.  With all blocks computed again the
 // backward of B16 H8 T1024 d_head 64 takes 590 µs, against 275 and the fp32 MFMA

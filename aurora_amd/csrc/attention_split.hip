@@ -24,7 +24,7 @@
 // Queries whose result is not finite, and blocks that met an infinity in a tile
 // or values too far apart for the scales, are computed again with the fp32 MFMA:
 // scores beyond 2^12; among 16 keys of V, 16 or more values (d_head if that is less:
-// as many as a row or a column has) that are not zero but 2^16 or more below the
+// as many as a row or a column has) that are not zero but 2^18 or more below the
 // tile's largest; a V that grows by more than 2^60 from the first tile on.  Fewer
 // small values than that keep an absolute error of 2^-40 of the tile's largest.
 // With all blocks computed again B16 H8 T1024 d_head 64 takes 380 µs, against 85

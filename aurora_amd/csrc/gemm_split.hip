@@ -27,11 +27,11 @@
 // shrinks when a later value would pass the limit; the accumulators of that row
 // are then rescaled before the next product is added.
 //
-// A value below 2^-2 at that scale, 2^15 … 2^18 below the row's largest, has an
-// absolute error of up to 2^-25 there instead of a relative one, which shows
-// where the row's large values meet zeros or small values of the column.  So the
-// values too small for their scale are counted per row and column (n and m): what
-// they can do to a result is at most E = (n + m)·2^-25·2^16.  It stands if E is
+// A value below 2^-2 at that scale has an absolute error of up to 2^-25 there
+// instead of a relative one, which shows where the row's large values meet zeros or
+// small values of the column.  Down to 2^-4 that is 2^-21 of the value.  The values
+// below, 2^17 … 2^20 below the row's largest, are counted per row and column (n and
+// m): what they can do to a result is at most E = (n + m)·2^-25·2^16.  It stands if E is
 // below 2^-21 of the sum of the products' magnitudes, for which there are two
 // lower bounds: the result's own magnitude, and, where the first 32 values of row
 // and column hold D and D' of 2^9 or more, (D + D' − 32)·2^18.  (That clears

@@ -30,10 +30,10 @@ __device__ __forceinline__ void split2(float x0, float x1, float s0, float s1, h
 }
 
 constexpr float kSplitLimit = 65504.f;  // largest scaled magnitude let through
-constexpr float kSplitFine = 0.25f;     // smallest that keeps its 23 bits
+constexpr float kSplitFine = 0.0625f;   // smallest whose error, 2^-25, is below 2^-21 of it
 
 // Is any |h| of N pairs outside [kSplitFine, kSplitLimit], zero, infinite or NaN?
-// (2h − 2·0x3400 in 16 bits, without the sign, is below 0x9000 for the others.)
+// (2h − 2·0x2c00 in 16 bits, without the sign, is below 0xa000 for the others.)
 typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
 template <int N>
 __device__ __forceinline__ ushort2v high_range(const half2v (&h)[N]) {
@@ -41,12 +41,12 @@ __device__ __forceinline__ ushort2v high_range(const half2v (&h)[N]) {
 #pragma unroll
   for (int e = 0; e < N; ++e) {
     ushort2v t;
-    asm("v_pk_mad_u16 %0, %1, 2, %2 op_sel_hi:[1,0,1]" : "=v"(t) : "v"(h[e]), "s"(0x98009800u));
+    asm("v_pk_mad_u16 %0, %1, 2, %2 op_sel_hi:[1,0,1]" : "=v"(t) : "v"(h[e]), "s"(0xa800a800u));
     m = __builtin_elementwise_max(m, t);
   }
   return m;
 }
-__device__ __forceinline__ bool out_of_range(ushort2v t) { return max(t[0], t[1]) >= 0x9000; }
+__device__ __forceinline__ bool out_of_range(ushort2v t) { return max(t[0], t[1]) >= 0xa000; }
 
 // Byte offset of granule q (8 k, 16 bytes) of row r in an LDS plane [ROWS][32]:
 // q ^ t(r / 4), t = 0, 2, 3, 1.  A b128 access runs in four phases of 16 lanes

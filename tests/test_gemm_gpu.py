@@ -581,8 +581,8 @@ def _wide_operands(name, m, n, k):
     elif name == "zeros":  # rows and columns of zeros, and zeros first
         a[::4], a[1::4, : k // 2], b[:, ::5], b[: k // 2, 1::5] = 0, 0, 0, 0
         a[2::4, k // 2 :] *= 2.0 ** -40
-    else:  # softmax gradient
-        p = np.exp(6 * a)
+    else:  # softmax gradient, of a trained model or at the start of training
+        p = np.exp((6 if name == "softmax" else 0.6) * a)
         a = p / p.sum(1, keepdims=True)
         a[np.arange(m), rng.integers(0, k, m)] -= 1
     return a.astype(np.float32), b.astype(np.float32)
@@ -590,13 +590,14 @@ def _wide_operands(name, m, n, k):
 
 @pytest.mark.parametrize("cfg", SPLIT_TILES)
 @pytest.mark.parametrize("name", ["outlier 8", "outlier 16", "outlier 24", "outlier 60", "ones", "late", "octets",
-                                  "reciprocal", "one-hot", "few", "zeros", "softmax"])
+                                  "reciprocal", "one-hot", "few", "zeros", "softmax", "softmax early"])
 def test_split_kernel_wide_rows(ctx, monkeypatch, cfg, name):
     """Values far below the largest of their row or column, where that meets zeros or
     small values: bound per element, in units of (|A||B|)_ij, that of
-    test_split_kernel_edges, (9 + K/32)·2^-24, and the 2^-21 that a result is let
-    stand at; what is computed again in fp32 rounds once a product, K·2^-24 at most
-    and √K·2^-24 usually.  Below 2e-6 for K = 333 all the same."""
+    test_split_kernel_edges, (9 + K/32)·2^-24, 2^-21 for values just large enough for
+    their scale, and the 2^-21 that a result is let stand at: 2.2e-6 for K = 333.  What
+    is computed again in fp32 rounds once a product, K·2^-24 at most and √K·2^-24
+    usually, which is less."""
     m, n, k = 150, 141, 333
     a, b = _wide_operands(name, m, n, k)
     a64, b64 = a.astype(np.float64), b.astype(np.float64)
@@ -608,7 +609,7 @@ def test_split_kernel_wide_rows(ctx, monkeypatch, cfg, name):
             if start is not None:
                 want, bound = want + start, bound + np.abs(start)
             err = np.abs(got - want)
-            assert np.all(err <= 2e-6 * bound + 2.0 ** -148), (cfg, name, ak, bk, splits, np.max(err / np.maximum(bound, 1e-300)))
+            assert np.all(err <= 2.2e-6 * bound + 2.0 ** -148), (cfg, name, ak, bk, splits, np.max(err / np.maximum(bound, 1e-300)))
 
 
 @pytest.mark.parametrize("cfg", SPLIT_TILES)
