@@ -34,9 +34,9 @@
 // m): what they can do to a result is at most E = (n + m)·2^-25·2^16.  It stands if E is
 // below 2^-21 of the sum of the products' magnitudes, for which there are two
 // lower bounds: the result's own magnitude, and, where the first 32 values of row
-// and column hold D and D' of 2^9 or more, (D + D' − 32)·2^18.  (That clears
-// N(0, 1) operands, halves of zeros and GELU outputs without a look at the
-// results.)  The others are computed again in fp32: a few of a wave as dot
+// and column hold D and D' of 2^9 or more, (D + D' − 32)·2^18, less by the bits that
+// the scales were lowered.  (That clears N(0, 1) operands, halves of zeros and GELU
+// outputs without a look at the results.)  The others are computed again in fp32: a few of a wave as dot
 // products, from more on the block's tile with the fp32 MFMA.  So is a tile with a
 // result that is not finite — an infinity or NaN among the operands, or a product
 // that overflows —, so that infinities and NaN come out as they do there.
@@ -72,7 +72,7 @@ typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
 // Scale exponent p of a row whose largest magnitude is m (0 when there is none
 // yet), and that of the factor 2^p.
 constexpr float kFineBound = 4096.f;    // |result| ≥ this · (n + m), at the scales: E ≤ 2^-21 of it
-constexpr int kDenseBound = 64;         // n + m ≤ this · (D + D' − 32): E ≤ 2^-21 of that bound
+constexpr int kDenseBound = 64;         // n + m ≤ this · (D + D' − 32): E ≤ 2^-21 of that bound (scales not lowered)
 constexpr int kZeroExp = 127;           // of a row of zeros so far, and of no other (but for values below 2^-111)
 __device__ __forceinline__ int row_exp(float m) {
   return m == 0.f ? kZeroExp : min(140 - (int)(__float_as_uint(m) >> 23), 126);
@@ -294,7 +294,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, BM == 64 ? 4 : 2) gemm_f16x3(G
   __shared__ int2 note[2][BM + BN];
   __shared__ int flag[2];
   // Of each row of A and column of B: the values too small for their scale; those
-  // of the first 32 that are large (0 once the scale was lowered) + 256·first scale
+  // of the first 32 that are large at the first scale, and 256 times its exponent
   __shared__ int fine[BM + BN], dense[BM + BN];
   __shared__ int rough;  // a result may have to be looked at
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -381,9 +381,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN, BM == 64 ? 4 : 2) gemm_f16x3(G
       note[(kt + 1) & 1][row] = int2{kt + 1, p - old};
       flag[(kt + 1) & 1] = kt + 1;
       if (op.koct == 0) {
-        const int p0 = old == kZeroExp ? p : dense[row] >> 8;
-        dense[row] = 256 * p0;
-        if (p < p0 - 60) atomicAdd(&fine[row], 1);
+        if (old == kZeroExp)
+          dense[row] = 256 * p;
+        else if (p < (dense[row] >> 8) - 60)
+          atomicAdd(&fine[row], 1);
       }
       op.set_exp(o, p);
     }
@@ -577,44 +578,49 @@ __global__ void __launch_bounds__(64 * WGM * WGN, BM == 64 ? 4 : 2) gemm_f16x3(G
   // The rows' and columns' final exponents, through the notes' memory.
   __syncthreads();
   int* ex = reinterpret_cast<int*>(&note[0][0]);
-  // > 0 for a row and a column together: their results are looked at
-  auto doubt = [&](int row) { return fine[row] - kDenseBound * ((dense[row] & 255) - 16); };
-  auto last = [&](auto& op, int o, int note0) {
-    const int row = note0 + op.row0 + op.step(o);
+  // The large values of a row and a column clear their result if n + m ≤
+  // 64·(D + D' − 32)·2^-(d + d'), with d the bits by which a scale was lowered; so they
+  // do if n ≤ 8·(D − 16)·2^-d and d ≤ 3 for both.  dense becomes D + 256·d.  Rows
+  // that are zero or past the operand are never in doubt.
+  constexpr int kNever = -(1 << 30);
+  auto last = [&](auto& op, int o, int note0, int rows) {
+    const int r = op.row0 + op.step(o), row = note0 + r;
     if (op.koct == 0) {
-      ex[row] = scale_exp(op.s[o]);
-      if (doubt(row) > 0 && ex[row] != kZeroExp) rough = 1;
+      const int p = scale_exp(op.s[o]), big = dense[row] & 255, d = min((dense[row] >> 8) - p, 15);
+      ex[row] = p;
+      dense[row] = big + 256 * d;
+      if (p == kZeroExp || r >= rows)
+        fine[row] = kNever;
+      else if (d > 3 || fine[row] > (kDenseBound / 8 * (big - 16)) >> d)
+        rough = 1;
     }
   };
 #pragma unroll
-  for (int o = 0; o < NOA; ++o) last(la, o, 0);
+  for (int o = 0; o < NOA; ++o) last(la, o, 0, g.M - m0);
 #pragma unroll
-  for (int o = 0; o < NOB; ++o) last(lb, o, BM);
+  for (int o = 0; o < NOB; ++o) last(lb, o, BM, g.N - n0);
   __syncthreads();
   int pc[TN];
   // Results to compute again: bit 4j + e of fl[i].
   unsigned fl[TM], worst = 0;
   int nfl = 0;
   if (rough) {
-    // A row or column of zeros, or past the operand, is never in doubt.
-    constexpr int kNever = -(1 << 30);
-    int dc[TN], nc[TN];
+    int nc[TN], wc[TN];
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      const int col = BM + wn * WN + 16 * j + l16;
-      nc[j] = fine[col];
-      dc[j] = ex[col] == kZeroExp || n0 + col - BM >= g.N ? kNever : doubt(col);
+      nc[j] = fine[BM + wn * WN + 16 * j + l16];
+      wc[j] = dense[BM + wn * WN + 16 * j + l16];
     }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       fl[i] = 0;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int row = wm * WM + 16 * i + 4 * g16 + e, nr = fine[row];
-        const int dr = ex[row] == kZeroExp || m0 + row >= g.M ? kNever : doubt(row);
+        const int row = wm * WM + 16 * i + 4 * g16 + e, nr = fine[row], wr = dense[row];
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-          const float bound = dr + dc[j] > 0 ? kFineBound * (float)(nr + nc[j]) : 0.f;
+          const int n = nr + nc[j], w = wr + wc[j], most = (kDenseBound * max((w & 255) - 32, 0)) >> (w >> 8);
+          const float bound = n > most ? kFineBound * (float)n : 0.f;
           fl[i] |= (fabsf(acc[i][j][e]) < bound ? 1u : 0u) << (4 * j + e);
         }
       }
