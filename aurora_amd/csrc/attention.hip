@@ -668,6 +668,8 @@ void launch_bwd(const aur_ctx* ctx, const AttnArgs& a, int b) {
   hipLaunchKernelGGL(mha_bwd_rowdot_kernel<DH>, dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256),
                      0, st, a, b);
   dim3 grid(a.H, b, (a.T + TQ - 1) / TQ);
+  // (AUR_ATTN_DKV_NS2, like AUR_ATTN_FWD_STAGED, chooses among the fp32 kernels: it
+  // has no say where the split ones run.)
   if (bwd_takes_split(ctx, (uint32_t)b, (uint32_t)a.T, (uint32_t)a.H, DH))
     bwd_dkv_split(a, b, DH, st);
   else if (std::getenv("AUR_ATTN_DKV_NS2") == nullptr)

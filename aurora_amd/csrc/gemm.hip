@@ -879,7 +879,8 @@ double split_tile_us(const SplitTile& t, long blocks, int cus, int nk, int k_str
 // admits the 256×128 tile (direct-load kernel only: whole tiles, aligned
 // operands, A k-contiguous — with A k-strided it measured 4 % slower than
 // 128×128 — and no prefetched epilogue operand): 1.03 relative efficiency,
-// 0.75 when alone on a CU.  Against the clock the modelled time stands for
+// 0.75 when alone on a CU; since the split-fp16 kernel takes the shapes it was made
+// for, it serves those of K = 32 and little else.  Against the clock the modelled time stands for
 // 2.1 µs + 1.17 × it on whole tiles, 1.23 × with edges, 2.3 × where the rows
 // allow no 16-byte loads (12 % rms on the same 100 shapes).
 //

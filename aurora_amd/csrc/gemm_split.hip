@@ -1,6 +1,6 @@
 // fp32 GEMM on the fp16 matrix cores: every fp32 operand value is split into
 // two fp16 numbers and the products are summed in fp32 by
-// v_mfma_f32_16x16x32_f16 (1.9 PFLOP/s with random operands in registers on
+// v_mfma_f32_16x16x32_f16 (1.8 PFLOP/s with random operands in registers on
 // MI355X, where power sets the clock, against 0.15 for the fp32 MFMA).
 //
 //   x·2^p = h + l,  h = fp16(x·2^p),  l = fp16(x·2^p − h)
@@ -18,8 +18,9 @@
 // are scaled by −2^p: the sign of that error alternates over the result.
 // Relative error against float64 on normal operands, fp32 MFMA → here: 1.4e-7
 // → 0.93e-7 at K = 64, 4.0e-7 → 1.2e-7 at 512, 1.16e-6 → 2.4e-7 at 4096,
-// 2.3e-6 → 4.4e-7 at 16384; the same order holds for uniform, all-positive,
-// softmax-gradient and widely scaled operands.
+// 2.3e-6 → 4.4e-7 at 16384; the same order holds for uniform, all-positive
+// and softmax-gradient operands; what is computed again in fp32 (below) has the fp32
+// MFMA's error.
 //
 // fp16 spans only 2^-24 … 2^16, so every row of A and column of B carries its
 // own power-of-two scale 2^p.  It starts from the row's first 32 values (their
@@ -44,13 +45,13 @@
 // What bounds it: per 32 of K a wave of the 256×256 tile (128×64 outputs)
 // issues 96 MFMAs (1536 matrix-core cycles), 128 additions, ≈ 150 operations
 // of splitting and checking, 24 fragment reads and 8 LDS writes, and the waves of a
-// SIMD hardly overlap the two; power holds the clock at 1.7-1.9 GHz.
-// Measured (fp32 MFMA kernels → here): A·Bᵀ 16384×1024×4096 970 → 390 µs (352
-// TFLOP/s), 8192×2048×512 129 → 60 µs, dW 4096×1024 over 16384 rows 1016 →
-// 437 µs, 777×1023×513 24.3 → 15.5 µs.  Counting the small values is 2 µs of each
-// but the last's 11 % (one wave per SIMD there).  Tiles that are computed again add
-// the fp32 MFMA's time: 4096×1024×4096 140 µs, all of it again (one outlier of 2^8
-// or more a row, met by zeros) 370 to 440, where the fp32 kernels take 255.
+// SIMD hardly overlap the two (matrix cores busy 53 % of the cycles).
+// Measured (fp32 MFMA kernels → here): A·B 16384×1024×4096 982 → 376 µs (365
+// TFLOP/s), 8192×2048×512 129 → 59 µs, dW 4096×1024 over 16384 rows 1016 →
+// 422 µs, 777×1023×513 24.3 → 14.9 µs.  Counting the small values is 2 µs of the
+// second and 1.3 of the last (one wave per SIMD there).  Tiles that are computed
+// again add the fp32 MFMA's time: 4096×1024×4096 140 µs, all of it again (an outlier
+// of 2^12 or more in a row, met by zeros) 370 to 440, where the fp32 kernels take 255.
 // The 256×256 tile needs the fewest LDS and L2 bytes per product; the
 // smaller tiles serve shapes with few output tiles (choose_plan in gemm.hip).
 #include "common.hpp"
