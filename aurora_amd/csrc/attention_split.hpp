@@ -15,8 +15,8 @@ struct SplitGeo {
   static constexpr int KROW = KS * 64;       // bytes of a K row in LDS
   static constexpr int KPLANE = 64 * KROW, VPLANE = DT * 16 * 128;
   // Small values among 16 rows of a tile that are one too many: a row of them has
-  // DH, a column 16.  (N(0, 1) values have 0.05 on average, those with
-  // columns 30 times the others' 1.)
+  // DH, a column 16.  (N(0, 1) values have 0.01 on average, those with
+  // columns 30 times the others' 0.3.)
   static constexpr int FINE = DH < 16 ? DH : 16;
 };
 
